@@ -356,12 +356,28 @@ static int split_contig(int prec, int lg, int* lg1, int* lg2) {
   // L = L1 (strided pass with the four-step twiddle) * L2 (contiguous pass);
   // 2^22 as 1024 x 4096 (the contiguous pass then runs four lines per CU and
   // three stages: 38.1 against 41.4 us for 512 x 8192)
-  const int mc = ilog2c(lmax_contig(prec)), ms = ilog2c(lmax_strided_fourstep(prec));
+  const int mc = ilog2c(lmax_contig(prec)), ms = prec == PREC_F32 ? 10 : 8;
   int b = std::min(mc, lg - 1);
   if (prec == PREC_F32 && lg == 22) b = 12;
   if (lg - b > ms) return -1;
   *lg2 = b;
   *lg1 = lg - b;
+  return 0;
+}
+
+// The same in natural order, L = L1 * L2: a strided pass over L1 that leaves
+// its lines contiguous, then a strided axis of L2 points at stride L1 whose
+// output is the natural order.  Both halves in one strided pass each while
+// they fit; FP32 2^21 and 2^22 keep two passes with the 4096-point column pass
+// for L2; longer axes run L2 as a strided four-step pair.  The limits are
+// those of the bit-reversed split.
+static int split_natural(int prec, int lg, int* lg1, int* lg2) {
+  const int m = ilog2c(lmax_strided_fourstep(prec));
+  if (split_contig(prec, lg, lg1, lg2)) return -1;
+  int a = std::min((lg + 1) / 2, m);
+  if (prec == PREC_F32 && (lg == 21 || lg == 22)) a = lg - 12;
+  *lg1 = a;
+  *lg2 = lg - a;
   return 0;
 }
 
@@ -386,6 +402,28 @@ static constexpr unsigned long long PLANE256_MIN_COUNT = 32;
 // plane pass): measured 29.5 against 31.2 us at 32 groups (4096 x 512), 39.9
 // against 32.9 us at 64 (4096 x 1024), 137.6 against 103.3 us at 4096 x 4096.
 static constexpr unsigned long long COL4096_MIN_GROUPS = 64;
+
+// split mode applies to lines with a radix-16 stage (16..4096 points)
+static bool line_split(bool split, int lg) { return split && lg >= 4 && lg <= 12; }
+// lines per workgroup of a line pass
+static int pass_cols(const PassDesc& p, bool split, int prec) {
+  return geom_cols_launch(1 << p.lg, p.mode, pass_kind(line_split(split, p.lg), prec), p.nouter * p.K * p.ncol);
+}
+
+// the 4096-point axis at element stride lx of `outer` arrays in one pass
+static PassDesc col4096_pass(long long lx, unsigned long long outer) {
+  PassDesc p;
+  p.lg = 12;
+  p.mode = MODE_COL4096;
+  p.transposing = true;  // the workgroups of a column group all read all of it
+  p.in_p = p.out_p = lx;
+  p.in_c = p.out_c = 1;
+  p.ncol = (unsigned)lx;
+  p.K = 1;
+  p.nouter = outer;
+  p.in_o = p.out_o = 4096 * lx;
+  return p;
+}
 
 static int build_plan(int rank, const size_t* dims, size_t batch, unsigned flags, int prec,
                       bool aliased, Plan& plan) {
@@ -471,20 +509,75 @@ static int build_plan(int rank, const size_t* dims, size_t batch, unsigned flags
     unsigned long long O = batch;
     for (int d = 0; d < rank - 2; ++d) O *= dims[d];
     if (col4096_supported(LX, O) && (unsigned long long)(LX / 16) * O >= COL4096_MIN_GROUPS) {
-      PassDesc p;
-      p.lg = 12;
-      p.mode = MODE_COL4096;
-      p.transposing = true;  // the four workgroups of a column group all read all of it
-      p.in_p = p.out_p = LX;
-      p.in_c = p.out_c = 1;
-      p.ncol = (unsigned)LX;
-      p.K = 1;
-      p.nouter = O;
-      p.in_o = p.out_o = 4096 * LX;
-      ps.push_back(p);
+      ps.push_back(col4096_pass(LX, O));
       col_axis = rank - 2;
     }
   }
+
+  // an axis of L points at element stride st (st > 1) of O arrays: one strided
+  // pass up to lmax points, the 4096-point column pass for the second half of
+  // a long contiguous axis (out of place), else a four-step pair
+  auto push_strided = [&](long long L, long long st, unsigned long long O, int lmax) -> int {
+    const int lg = ilog2c(L);
+    if (L <= lmax) {
+      PassDesc p;
+      p.lg = lg;
+      p.mode = MODE_STRIDED;
+      p.in_p = p.out_p = st;
+      p.in_c = p.out_c = 1;
+      if (st >= (1LL << 32)) {
+        set_error("axis stride too large");
+        return -1;
+      }
+      p.ncol = (unsigned)st;
+      p.nouter = O;
+      p.in_o = p.out_o = L * st;
+      ps.push_back(p);
+      return 0;
+    }
+    if (lmax > lmax_strided(prec) && L == 4096 && prec == PREC_F32 && !plan.split &&
+        !(flags & FLAG_NO_PLANE_FUSION) && col4096_supported(st, O)) {
+      ps.push_back(col4096_pass(st, O));
+      return 0;
+    }
+    int lg1, lg2;
+    if (split_strided(prec, lg, &lg1, &lg2)) {
+      set_error("strided axis of 2^%d points exceeds the supported length", lg);
+      return -1;
+    }
+    const long long L1 = 1LL << lg1, L2 = 1LL << lg2;
+    if (L2 * st >= (1LL << 32)) {
+      set_error("axis stride too large");
+      return -1;
+    }
+    PassDesc A;
+    A.lg = lg1;
+    A.mode = MODE_STRIDED;
+    A.epi = EPI_TWIDDLE;
+    A.in_p = A.out_p = L2 * st;
+    A.in_c = A.out_c = 1;
+    A.ncol = (unsigned)(L2 * st);
+    A.nouter = O;
+    A.in_o = A.out_o = L * st;
+    A.M = L;
+    A.cshift = (unsigned)ilog2c(st);
+    ps.push_back(A);
+    PassDesc B;
+    B.lg = lg2;
+    B.mode = MODE_STRIDED;
+    B.transposing = true;
+    B.in_p = st;
+    B.out_p = L1 * st;
+    B.in_c = B.out_c = 1;
+    B.ncol = (unsigned)st;
+    B.K = (unsigned)L1;
+    B.in_k = L2 * st;
+    B.out_k = st;
+    B.nouter = O;
+    B.in_o = B.out_o = L * st;
+    ps.push_back(B);
+    return 0;
+  };
 
   for (int a = top; a >= 0; --a) {
     const long long L = (long long)dims[a];
@@ -510,12 +603,12 @@ static int build_plan(int rank, const size_t* dims, size_t batch, unsigned flags
         ps.push_back(p);
       } else {
         int lg1, lg2;
-        if (split_contig(prec, lg, &lg1, &lg2)) {
+        if ((bitrev ? split_contig(prec, lg, &lg1, &lg2) : split_natural(prec, lg, &lg1, &lg2))) {
           set_error("contiguous axis of 2^%d points exceeds the supported length", lg);
           return -1;
         }
         const long long L1 = 1LL << lg1, L2 = 1LL << lg2;
-        PassDesc A;  // strided DFT over n1, post-twiddle W_L^{n2 k1}, in place
+        PassDesc A;  // strided DFT over n1, post-twiddle W_L^{n2 k1}
         A.lg = lg1;
         A.mode = MODE_STRIDED;
         A.epi = EPI_TWIDDLE;
@@ -526,88 +619,39 @@ static int build_plan(int rank, const size_t* dims, size_t batch, unsigned flags
         A.in_o = A.out_o = L;
         A.M = L;
         A.cshift = 0;
-        ps.push_back(A);
+        if (!bitrev) {
+          // line n2 leaves the pass as the contiguous run Z[n2][k1]; the DFT
+          // over n2 at stride L1 then ends in natural order, X[k1 + L1 k2] in
+          // place, in whole 128-byte segments (a contiguous pass over n2 whose
+          // store scattered single points took 47.9 of 60.2 us for 3 x 2^20)
+          A.out_p = 1;
+          A.out_c = L1;
+          A.transposing = true;
+          ps.push_back(A);
+          if (push_strided(L2, L1, O, lmax_strided_fourstep(prec))) return -1;
+          continue;
+        }
+        ps.push_back(A);  // in place
         PassDesc B;  // contiguous DFT over n2 for every k1
         B.lg = lg2;
         B.mode = MODE_CONTIG;
         B.transposing = true;
-        B.in_p = 1;
-        B.in_c = L2;
-        B.ncol = (unsigned)L1;
         B.nouter = O;
         B.in_o = B.out_o = L;
-        if (bitrev) {  // out[bitrev(k1)*L2 + bitrev(k2)] = X[k1 + L1 k2]
-          B.epi = EPI_BITREV;
-          B.out_p = 1;
-          B.out_c = L2;
-          B.K = 1;
-          // column bit reversal is expressed through the middle index: one column per K
-          B.ncol = 1;
-          B.K = (unsigned)L1;
-          B.in_k = L2;
-          B.out_k = L2;
-          B.in_c = B.out_c = 0;
-          B.kbits = (unsigned)lg1;
-        } else {  // X[k1 + L1 k2] at natural position (strided store)
-          B.epi = EPI_NONE;
-          B.out_p = L1;
-          B.out_c = 1;
-        }
+        // out[bitrev(k1)*L2 + bitrev(k2)] = X[k1 + L1 k2]: column bit reversal is
+        // expressed through the middle index, one column per K
+        B.epi = EPI_BITREV;
+        B.in_p = B.out_p = 1;
+        B.ncol = 1;
+        B.K = (unsigned)L1;
+        B.in_k = L2;
+        B.out_k = L2;
+        B.in_c = B.out_c = 0;
+        B.kbits = (unsigned)lg1;
         ps.push_back(B);
       }
     } else {
-      if (L <= lmax_strided(prec)) {
-        PassDesc p;
-        p.lg = lg;
-        p.mode = MODE_STRIDED;
-        p.in_p = p.out_p = s;
-        p.in_c = p.out_c = 1;
-        if (s >= (1LL << 32)) {
-          set_error("axis stride too large");
-          return -1;
-        }
-        p.ncol = (unsigned)s;
-        p.nouter = O;
-        p.in_o = p.out_o = L * s;
-        ps.push_back(p);
-      } else {
-        int lg1, lg2;
-        if (split_strided(prec, lg, &lg1, &lg2)) {
-          set_error("strided axis of 2^%d points exceeds the supported length", lg);
-          return -1;
-        }
-        const long long L1 = 1LL << lg1, L2 = 1LL << lg2;
-        if (L2 * s >= (1LL << 32)) {
-          set_error("axis stride too large");
-          return -1;
-        }
-        PassDesc A;
-        A.lg = lg1;
-        A.mode = MODE_STRIDED;
-        A.epi = EPI_TWIDDLE;
-        A.in_p = A.out_p = L2 * s;
-        A.in_c = A.out_c = 1;
-        A.ncol = (unsigned)(L2 * s);
-        A.nouter = O;
-        A.in_o = A.out_o = L * s;
-        A.M = L;
-        A.cshift = (unsigned)ilog2c(s);
-        ps.push_back(A);
-        PassDesc B;
-        B.lg = lg2;
-        B.mode = MODE_STRIDED;
-        B.transposing = true;
-        B.in_p = s;
-        B.out_p = L1 * s;
-        B.in_c = B.out_c = 1;
-        B.ncol = (unsigned)s;
-        B.K = (unsigned)L1;
-        B.in_k = L2 * s;
-        B.out_k = s;
-        B.nouter = O;
-        B.in_o = B.out_o = L * s;
-        ps.push_back(B);
-      }
+      if (push_strided(L, s, O, lmax_strided(prec))) return -1;
     }
   }
 
@@ -867,9 +911,9 @@ static int run_plan(Plan& plan, const void* din, void* dout, bool inverse, hipSt
     a.out_o = p.out_o;
     a.ncol = p.ncol;
     const int L = 1 << p.lg;
-    // split mode applies to lines with a radix-16 stage (16..4096 points)
-    const bool split = plan.split && L >= 16 && L <= 4096;
-    const int C = geom_cols_for(L, p.mode, split);
+    const bool split = line_split(plan.split, p.lg);
+    const int C = pass_cols(p, plan.split, plan.prec);
+    a.cols = C;
     a.ncb = (p.ncol + C - 1) / C;
     a.K = p.K;
     a.kbits = p.kbits;
@@ -884,7 +928,7 @@ static int run_plan(Plan& plan, const void* din, void* dout, bool inverse, hipSt
       a.ptw_cshift = p.cshift;
     }
     const unsigned long long per_outer = (unsigned long long)a.ncb * a.K;
-    const unsigned long long max_blocks = (0xFFFFFFFFULL / (unsigned)geom_threads_for(L, p.mode, split));
+    const unsigned long long max_blocks = (0xFFFFFFFFULL / (unsigned)(C * geom_tpl(L)));
     const unsigned long long outer_per_launch = std::max(1ULL, max_blocks / per_outer);
     for (unsigned long long o0 = 0; o0 < p.nouter; o0 += outer_per_launch) {
       const unsigned long long no = std::min(outer_per_launch, p.nouter - o0);
@@ -1399,7 +1443,7 @@ static int group_plane_args(const MultiPlan* mp, const PlaneGroup& g, PlaneArgs*
   z.in_p = z.out_p = s;
   z.in_c = z.out_c = 1;
   z.ncol = (unsigned)s;
-  const int zc = geom_cols_for((int)L, MODE_STRIDED, mp->split && L >= 16);
+  const int zc = geom_cols_for((int)L, MODE_STRIDED, pass_kind(mp->split && L >= 16, PREC_F32));
   z.ncb = (unsigned)((s + zc - 1) / zc);
   z.K = 1;
   z.inverse = mp->inverse ? 1 : 0;
@@ -1904,7 +1948,6 @@ int describe_plan(int rank, const size_t* dims, size_t batch, unsigned flags, in
     set_error("describe_plan: buffer too small");
     return -1;
   }
-  auto sp = [&](const PassDesc& d) { return p.split && d.lg >= 4 && d.lg <= 12; };
   // threads per workgroup of a plane pass: 512 for 256 x 256 (four per plane)
   // and for FP32 128 x 128 (two halves), LY * LX / 16 otherwise
   auto plane_threads = [&](const PassDesc& d) -> long long {
@@ -1921,12 +1964,12 @@ int describe_plan(int rank, const size_t* dims, size_t batch, unsigned flags, in
                        : d.mode == MODE_COL4096 ? 16
                        : d.mode == MODE_CUBE_A ? (d.lg == 9 ? 64 : (1LL << d.lg) / 4)   // rows per workgroup
                        : d.mode == MODE_CUBE_B ? (d.lg == 9 ? 8 : d.lg == 8 ? 16 : 32)   // columns per workgroup (x 8 or 4 rows x n planes)
-                       : geom_cols_for(1 << d.lg, d.mode, sp(d)),
+                       : pass_cols(d, p.split, prec),
                        d.mode == MODE_PLANE ? plane_threads(d)
                        : d.mode == MODE_COL4096 ? 512
                        : d.mode == MODE_CUBE_A ? (d.lg == 9 ? 1024 : d.lg == 8 ? 512 : 256)
                        : d.mode == MODE_CUBE_B ? (d.lg == 9 ? 1024 : 512)
-                       : geom_threads_for(1 << d.lg, d.mode, sp(d))};
+                       : pass_cols(d, p.split, prec) * geom_tpl(1 << d.lg)};
     for (int k = 0; k < NF; ++k) f[k] = v[k];
   }
   out[NF * n] = p.final_copy ? 1 : 0;

@@ -24,6 +24,7 @@ struct PassArgs {
   unsigned ptw_mmask;
   unsigned ptw_cshift;
   int inverse;
+  int cols;               // lines per workgroup (ncb counts those; 0: geom_cols_for())
   // optional real weights, one per point of a transform (broadcast over the
   // batch): the input is multiplied by w_load[e & w_mask] when read, the
   // output by w_store[e & w_mask] when written (e = element offset)

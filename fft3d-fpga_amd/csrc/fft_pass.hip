@@ -19,27 +19,41 @@
 
 namespace fftamd {
 
-template <typename R, int L, int MODE, int EPI, bool SPLIT, int DIR>
-__global__ void __launch_bounds__(geom_threads_for(L, MODE, SPLIT))
-    k_fft_pass(const PassArgs a) {
-  constexpr int CC = geom_cols_for(L, MODE, SPLIT);
+template <typename R>
+constexpr int kind_of(bool split) { return pass_kind(split, sizeof(R) == 4 ? PREC_F32 : PREC_F64); }
+
+template <typename R, int L, int MODE, int EPI, bool SPLIT, int DIR, int CC>
+__global__ void __launch_bounds__(CC * geom_tpl(L)) k_fft_pass(const PassArgs a) {
   using G = Geom<L, MODE, CC>;
-  constexpr bool NEED_LDS = G::NP > 1;
+  constexpr bool NEED_LDS = G::NP > 1 || EPI == EPI_TWIDDLE_T;
   __shared__ cpx<R> lds[NEED_LDS ? G::LDS_ELEMS : 1];
   pass_block<R, L, MODE, EPI, SPLIT, DIR, CC>(a, blockIdx.x, lds, (int)threadIdx.x);
 }
 
 // ---- launch table ------------------------------------------------------------
 
+template <typename R, int MODE, int EPI, int L, bool SPLIT, int CC>
+static void launch_cc(const PassArgs& a, unsigned long long blocks, hipStream_t s) {
+  // one kernel per direction: the direction swaps become register renames
+  constexpr int NT = CC * geom_tpl(L);
+  if (a.inverse)
+    FFTAMD_LAUNCH((k_fft_pass<R, L, MODE, EPI, SPLIT, 1, CC>), dim3((unsigned)blocks), dim3(NT), 0, s, a);
+  else
+    FFTAMD_LAUNCH((k_fft_pass<R, L, MODE, EPI, SPLIT, 0, CC>), dim3((unsigned)blocks), dim3(NT), 0, s, a);
+}
+
 template <typename R, int MODE, int EPI, int LG, bool SPLIT>
 static void launch_one(const PassArgs& a, unsigned long long blocks, hipStream_t s) {
   constexpr int L = 1 << LG;
-  // one kernel per direction: the direction swaps become register renames
-  constexpr int NT = geom_threads_for(L, MODE, SPLIT);
-  if (a.inverse)
-    FFTAMD_LAUNCH((k_fft_pass<R, L, MODE, EPI, SPLIT, 1>), dim3((unsigned)blocks), dim3(NT), 0, s, a);
-  else
-    FFTAMD_LAUNCH((k_fft_pass<R, L, MODE, EPI, SPLIT, 0>), dim3((unsigned)blocks), dim3(NT), 0, s, a);
+  constexpr int KIND = kind_of<R>(SPLIT);
+  constexpr int mid = geom_cols_mid(L, MODE, KIND), tiny = geom_cols_tiny(L, MODE, KIND);
+  if constexpr (mid != 0) {
+    if (a.cols == mid) return launch_cc<R, MODE, EPI, L, SPLIT, mid>(a, blocks, s);
+  }
+  if constexpr (tiny != 0) {
+    if (a.cols == tiny) return launch_cc<R, MODE, EPI, L, SPLIT, tiny>(a, blocks, s);
+  }
+  launch_cc<R, MODE, EPI, L, SPLIT, geom_cols_for(L, MODE, KIND)>(a, blocks, s);
 }
 
 template <typename R, int MODE, int EPI, int LG, bool SPLIT>
@@ -54,8 +68,8 @@ static bool dispatch_lg(int lg, const PassArgs& a, unsigned long long blocks, hi
       constexpr bool split_ok = !SPLIT || (sizeof(R) == 4 && L >= 16 && L <= 4096);
       constexpr bool ok = split_ok &&
                           (MODE == MODE_CONTIG ? L <= lmax_contig(prec)
-                                                : L <= (EPI == EPI_TWIDDLE ? lmax_strided_fourstep(prec)
-                                                                           : lmax_strided(prec))) &&
+                                                : L <= (EPI == EPI_TWIDDLE && prec == PREC_F64 ? lmax_strided(prec)
+                                                                                               : lmax_strided_fourstep(prec))) &&
                           !(MODE == MODE_CONTIG && EPI == EPI_TWIDDLE) &&
                           !(MODE == MODE_STRIDED && EPI == EPI_BITREV);
       if constexpr (ok) {
@@ -77,16 +91,19 @@ static bool dispatch_prec(int lg, int mode, int epi, const PassArgs& a, unsigned
     if (epi == EPI_BITREV) return dispatch_lg<R, MODE_CONTIG, EPI_BITREV, 1, SPLIT>(lg, a, blocks, s);
   } else {
     if (epi == EPI_NONE) return dispatch_lg<R, MODE_STRIDED, EPI_NONE, 1, SPLIT>(lg, a, blocks, s);
-    if (epi == EPI_TWIDDLE) return dispatch_lg<R, MODE_STRIDED, EPI_TWIDDLE, 1, SPLIT>(lg, a, blocks, s);
+    if (epi == EPI_TWIDDLE)
+      return a.out_p == 1 ? dispatch_lg<R, MODE_STRIDED, EPI_TWIDDLE_T, 1, SPLIT>(lg, a, blocks, s)
+                          : dispatch_lg<R, MODE_STRIDED, EPI_TWIDDLE, 1, SPLIT>(lg, a, blocks, s);
   }
   return false;
 }
 
-void preload_pass() { preload_kernel(reinterpret_cast<const void*>(&k_fft_pass<float, 256, MODE_CONTIG, EPI_NONE, false, 0>)); }
+void preload_pass() { preload_kernel(reinterpret_cast<const void*>(&k_fft_pass<float, 256, MODE_CONTIG, EPI_NONE, false, 0, geom_cols(256, MODE_CONTIG)>)); }
 
 int launch_fft_pass(int prec, int lg, int mode, int epi, const PassArgs& a, unsigned long long blocks,
                     void* stream, bool split) {
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  if (epi == EPI_TWIDDLE && a.out_p == 1 && a.w_store) return -1;  // the transposed store takes no weights
   bool ok;
   if (prec == PREC_F32)
     ok = split ? dispatch_prec<float, true>(lg, mode, epi, a, blocks, s)

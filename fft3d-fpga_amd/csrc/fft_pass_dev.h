@@ -267,6 +267,8 @@ __device__ __forceinline__ void tile_finish(const PassArgs& a, const TileLoc& t,
       }
     }
   } else {
+    constexpr bool TW = EPI == EPI_TWIDDLE || EPI == EPI_TWIDDLE_T;
+    if constexpr (EPI == EPI_TWIDDLE_T && NP > 1) __syncthreads();  // the last stage has read its inputs
 #pragma unroll
     for (int b = 0; b < NBL; ++b) {
       const int j = tau + b * TPL;
@@ -274,7 +276,7 @@ __device__ __forceinline__ void tile_finish(const PassArgs& a, const TileLoc& t,
       // k = j + r*NSL: W^{cc j} times the table powers W^{cc NSL m}, m = 1, 2,
       // 4, 8 (each from the two-level table: two loads and one product)
       cpx<R> base{}, s1{}, s2{}, s4{}, s8{};
-      if constexpr (EPI == EPI_TWIDDLE) {
+      if constexpr (TW) {
         const unsigned cc = col >> a.ptw_cshift;
         const cpx<R>* lo = reinterpret_cast<const cpx<R>*>(a.ptw_lo);
         const cpx<R>* hi = reinterpret_cast<const cpx<R>*>(a.ptw_hi);
@@ -294,7 +296,7 @@ __device__ __forceinline__ void tile_finish(const PassArgs& a, const TileLoc& t,
       for (int r = 0; r < RL; ++r) {
         const int k = j + r * NSL;
         cpx<R> x = v[b * RL + r];
-        if constexpr (EPI == EPI_TWIDDLE) {
+        if constexpr (TW) {
           cpx<R> w = base;
           if (r & 1) w = cmul(w, s1);
           if (r & 2) w = cmul(w, s2);
@@ -303,10 +305,27 @@ __device__ __forceinline__ void tile_finish(const PassArgs& a, const TileLoc& t,
           x = cmul(x, w);
         }
         if (inv) x = cswap(x);
-        if (active) {
+        if constexpr (EPI == EPI_TWIDDLE_T) {
+          lds[G::idx(c, k)] = x;
+        } else if (active) {
           if (a.w_store) x = cscale(x, (R)a.w_store[(unsigned long long)(out_off + (long long)k * a.out_p) & a.w_mask]);
           out[(long long)k * a.out_p] = x;
         }
+      }
+    }
+    if constexpr (EPI == EPI_TWIDDLE_T) {
+      // the tile leaves LDS line by line, adjacent threads on adjacent points:
+      // each line is one contiguous run of the output (never a plan's last
+      // pass, so it takes no store weights)
+      static_assert(MODE == MODE_STRIDED, "contiguous lines need no transposed store");
+      __syncthreads();
+      cpx<R>* __restrict__ tile = out - (long long)c * a.out_c;
+      const unsigned col0 = col - (unsigned)c;
+      const int t0 = tau * G::C + c;  // thread index within the tile
+#pragma unroll
+      for (int i = 0; i < PPT; ++i) {
+        const int e = t0 + i * G::NT, q = e / L, p = e % L;
+        if (col0 + (unsigned)q < a.ncol) tile[(long long)q * a.out_c + p] = lds[G::idx(q, p)];
       }
     }
   }

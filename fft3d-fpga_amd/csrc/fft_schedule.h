@@ -19,7 +19,9 @@ enum PassMode { MODE_CONTIG = 0, MODE_STRIDED = 1, MODE_PLANE = 2, MODE_COL4096 
                 MODE_CUBE_B = 5 };
 // EPI_TWIDDLE multiplies point k of column c by W_M^{(c >> cshift) * k}
 // (four-step split of a long axis); EPI_BITREV stores point k at bitrev(k).
-enum PassEpilogue { EPI_NONE = 0, EPI_TWIDDLE = 1, EPI_BITREV = 2 };
+// EPI_TWIDDLE_T is EPI_TWIDDLE of a strided pass whose output lines are
+// contiguous (out_p == 1): the launcher picks it, a plan says EPI_TWIDDLE.
+enum PassEpilogue { EPI_NONE = 0, EPI_TWIDDLE = 1, EPI_BITREV = 2, EPI_TWIDDLE_T = 3 };
 enum Precision { PREC_F32 = 0, PREC_F64 = 1 };
 
 constexpr int ilog2c(long long x) { return x <= 1 ? 0 : 1 + ilog2c(x >> 1); }
@@ -60,23 +62,51 @@ constexpr int geom_cols(int L, int mode) {
                              : (L >= 1024 ? 16 : L >= 512 ? 32 : L >= 256 ? 16 : 256 / geom_tpl(L));
 }
 constexpr int geom_threads(int L, int mode) { return geom_cols(L, mode) * geom_tpl(L); }
-// Columns per workgroup of a line pass in either precision mode: split-
-// precision strided lines of 512 points and more keep 16 columns (two
-// workgroups per CU; with the FP32 layout's 32 columns, one, the split 512^3
-// line passes took 1.80 against 1.59 ms).
-constexpr int geom_cols_for(int L, int mode, bool split) {
-  return split && mode == MODE_STRIDED && L >= 512 ? 16 : geom_cols(L, mode);
+// Lines per workgroup of a line pass by the kind of its stages.  Strided lines
+// of 512 points and more: split precision keeps 16 columns (two workgroups per
+// CU; with the FP32 layout's 32 columns, one, the split 512^3 line passes took
+// 1.80 against 1.59 ms), FP64 8 (128-byte segments; 1024 points are 144 KiB of
+// LDS).
+enum PassKind { KIND_F32 = 0, KIND_SPLIT = 1, KIND_F64 = 2 };
+constexpr int pass_kind(bool split, int prec) { return split ? KIND_SPLIT : prec == PREC_F64 ? KIND_F64 : KIND_F32; }
+constexpr int geom_cols_for(int L, int mode, int kind) {
+  return mode == MODE_STRIDED && L >= 512 && kind != KIND_F32 ? (kind == KIND_SPLIT ? 16 : 8) : geom_cols(L, mode);
 }
-constexpr int geom_threads_for(int L, int mode, bool split) { return geom_cols_for(L, mode, split) * geom_tpl(L); }
+// Smaller tiles for a launch whose usual ones would leave CUs idle: `mid`, one
+// wave or 16 strided columns, and `tiny`, 8 strided columns (64-byte segments),
+// 0 where the kind of line has none.
+constexpr int geom_wave_lines(int L) { return geom_tpl(L) >= 64 ? 1 : 64 / geom_tpl(L); }
+constexpr int geom_cols_mid(int L, int mode, int kind) {
+  const int c = mode == MODE_CONTIG || geom_wave_lines(L) > 16 ? geom_wave_lines(L) : 16;
+  return kind != KIND_SPLIT && c < geom_cols_for(L, mode, kind) ? c : 0;
+}
+constexpr int geom_cols_tiny(int L, int mode, int kind) {
+  return kind != KIND_SPLIT && mode == MODE_STRIDED && geom_wave_lines(L) <= 8 && geom_cols_for(L, mode, kind) > 8 ? 8
+                                                                                                                  : 0;
+}
+// Lines per workgroup of a launch of `lines` lines: `mid` where the usual tile
+// gives at most half of the 256 CUs a workgroup, then `tiny` below 64 workgroups.
+// Measured for both passes of natural-order 1D transforms: 2^18 points (16
+// workgroups of 32 columns) 20.9 us, of 8 columns 14.2; 2^21 (128 of 32 in its
+// first pass) 37.3 us, of 16 columns 35.2; 12 x 2^18 (192 of 32) 29.1 us, of 16
+// columns 30.0, of 8 36.0; 2^20 (64 of 16) 25.0 us, of 8 24.6; 3 x 2^20 (192 of
+// 16) 29.1 us, of 8 36.8.  Contiguous 1024-point lines, 100 of them (25
+// workgroups of four): 10.9 us, one per workgroup 9.8.
+constexpr int geom_cols_launch(int L, int mode, int kind, unsigned long long lines) {
+  int c = geom_cols_for(L, mode, kind);
+  const int mid = geom_cols_mid(L, mode, kind), tiny = geom_cols_tiny(L, mode, kind);
+  if (mid && lines <= 128ull * (unsigned)c) c = mid;
+  if (tiny && lines < 64ull * (unsigned)c) c = tiny;
+  return c;
+}
 
 // Largest line held by one workgroup (LDS budget).  Longer axes are split
 // four-step into two passes.
 constexpr int lmax_contig(int prec) { return prec == PREC_F32 ? 8192 : 4096; }
 constexpr int lmax_strided(int prec) { return prec == PREC_F32 ? 512 : 256; }
-// The strided (first) pass of a four-step split of a long contiguous axis may
-// hold 1024-point lines (16 columns, 1024 threads, 139 KiB of LDS): 2^22 points
-// as 1024 x 4096 measured 38.1 against 41.4 us for 512 x 8192.  Strided axes
-// of 2D and 3D arrays keep lmax_strided.
-constexpr int lmax_strided_fourstep(int prec) { return prec == PREC_F32 ? 1024 : 256; }
+// The strided passes of a four-step split of a long contiguous axis may hold
+// 1024 points (16 columns FP32, 8 FP64, 139-144 KiB of LDS): 2^22 points as
+// 1024 x 4096 measured 38.1 against 41.4 us for 512 x 8192.
+constexpr int lmax_strided_fourstep(int) { return 1024; }
 
 }  // namespace fftamd
