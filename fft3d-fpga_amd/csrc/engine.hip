@@ -111,7 +111,7 @@ struct State {
   std::map<PlanKey, Plan> plans;
   std::map<std::pair<int, int>, void*> tw_stockham;  // (prec, L)
   std::map<std::pair<int, long long>, std::pair<void*, void*>> tw_fourstep;  // (prec, M)
-  std::map<long long, void*> tw_direct;  // FP32 W_M^t, t = 0..M-1
+  std::map<std::pair<int, long long>, void*> tw_direct;  // (prec, M): W_M^t, t = 0..M-1
   // bumped whenever tables and plans are released (fpga_final, re-init):
   // multi-transform plans and graphs made before hold freed table pointers
   unsigned long long gen = 1;
@@ -253,22 +253,29 @@ static int get_fourstep(int prec, long long M, const void** lo, const void** hi)
   return 0;
 }
 
-// FP32 table of W_M^t for every t < M (one load per twiddle)
-static int get_direct(long long M, const void** out) {
+// table of W_M^t for every t < M (one load per twiddle)
+template <typename R>
+static int make_direct(long long M, void** d) {
+  std::vector<R> h(2 * (size_t)M);
+  for (long long t = 0; t < M; ++t) {
+    long double c, s;
+    twiddle_ld(t, M, &c, &s);
+    h[2 * t] = (R)c;
+    h[2 * t + 1] = (R)s;
+  }
+  HIP_TRY(hipMalloc(d, h.size() * sizeof(R)));
+  HIP_TRY(hipMemcpy(*d, h.data(), h.size() * sizeof(R), hipMemcpyHostToDevice));
+  return 0;
+}
+
+static int get_direct(long long M, const void** out, int prec = PREC_F32) {
   State& st = S();
-  auto it = st.tw_direct.find(M);
+  const auto key = std::make_pair(prec, M);
+  auto it = st.tw_direct.find(key);
   if (it == st.tw_direct.end()) {
-    std::vector<float> h(2 * (size_t)M);
-    for (long long t = 0; t < M; ++t) {
-      long double c, s;
-      twiddle_ld(t, M, &c, &s);
-      h[2 * t] = (float)c;
-      h[2 * t + 1] = (float)s;
-    }
     void* d = nullptr;
-    HIP_TRY(hipMalloc(&d, h.size() * sizeof(float)));
-    HIP_TRY(hipMemcpy(d, h.data(), h.size() * sizeof(float), hipMemcpyHostToDevice));
-    it = st.tw_direct.emplace(M, d).first;
+    if (prec == PREC_F32 ? make_direct<float>(M, &d) : make_direct<double>(M, &d)) return -1;
+    it = st.tw_direct.emplace(key, d).first;
   }
   *out = it->second;
   return 0;
@@ -397,6 +404,8 @@ static int split_strided(int prec, int lg, int* lg1, int* lg2) {
 // measured 13.9 against 16.9 us at 16 planes, 20.6 against 18.1 at 32).
 static constexpr unsigned long long PLANE_MIN_COUNT = 1;
 static constexpr unsigned long long PLANE256_MIN_COUNT = 32;
+// most planes of one launch (grid size in work-items is 32-bit)
+static constexpr unsigned long long PLANE_MAX_COUNT = 0xFFFFFFFFull / 1024;
 // Fewest 16-column groups for which the one-pass 4096-point column transform
 // replaces the four-step pair (four workgroups per group, as the 256 x 256
 // plane pass): measured 29.5 against 31.2 us at 32 groups (4096 x 512), 39.9
@@ -447,8 +456,10 @@ static int build_plan(int rank, const size_t* dims, size_t batch, unsigned flags
   // stage and z (in place)
   int top = rank - 1;
   const long long CN = rank >= 3 ? (long long)dims[rank - 1] : 0;
-  if (rank >= 3 && prec == PREC_F32 && !(flags & (FLAG_NO_PLANE_FUSION | FLAG_NO_CUBE_SPLIT)) &&
-      (CN == 512 || CN == 256 || CN == 128) && (long long)dims[rank - 2] == CN && (long long)dims[rank - 3] == CN) {
+  // FP64: 128^3 only, and out of place (in place the pair would need a
+  // temporary buffer that the line passes do not)
+  if (rank >= 3 && !(flags & (FLAG_NO_PLANE_FUSION | FLAG_NO_CUBE_SPLIT)) &&
+      (prec == PREC_F32 ? CN == 512 || CN == 256 || CN == 128 : CN == 128 && !aliased) && (long long)dims[rank - 2] == CN && (long long)dims[rank - 3] == CN) {
     unsigned long long O = batch;
     for (int d = 0; d < rank - 3; ++d) O *= dims[d];
     PassDesc A;
@@ -477,13 +488,13 @@ static int build_plan(int rank, const size_t* dims, size_t batch, unsigned flags
   // planes of the two fastest axes in one fused x+y pass: 256 x 256 (four
   // workgroups per plane, out of place) or up to 128 x 128 (one workgroup
   // per plane in LDS, in place allowed)
-  if (top == rank - 1 && rank >= 2 && prec == PREC_F32 && !(flags & FLAG_NO_PLANE_FUSION)) {
+  if (top == rank - 1 && rank >= 2 && !(flags & FLAG_NO_PLANE_FUSION)) {
     const long long LY = (long long)dims[rank - 2], LX = (long long)dims[rank - 1];
     unsigned long long O = batch;
     for (int d = 0; d < rank - 2; ++d) O *= dims[d];
-    const bool big = LY == 256 && LX == 256;  // no split-precision variant
+    const bool big = prec == PREC_F32 && LY == 256 && LX == 256;  // no split-precision variant
     if ((big && !plan.split && O >= PLANE256_MIN_COUNT) ||
-        (plane_shape_supported(LY, LX) && O >= PLANE_MIN_COUNT)) {
+        (plane_shape_supported(LY, LX, prec) && O >= PLANE_MIN_COUNT && (prec == PREC_F32 || O <= PLANE_MAX_COUNT))) {
       PassDesc p;
       p.lg = ilog2c(LX);
       p.mode = MODE_PLANE;
@@ -717,7 +728,7 @@ static int tab_fourstep(const Plan& plan, long long M, const void** lo, const vo
   return 0;
 }
 static int tab_direct(const Plan& plan, long long M, const void** out) {
-  if (!plan.noalloc) return get_direct(M, out);
+  if (!plan.noalloc) return get_direct(M, out, plan.prec);
   const NoallocDev& d = na_dev[S().dev];
   if (!d.ready || (M != 256 && M != 512)) {
     set_error("no allocation-free table of W_%lld", M);
@@ -812,11 +823,12 @@ static int run_plan(Plan& plan, const void* din, void* dout, bool inverse, hipSt
       const bool prof = pf.on && !resolve && pf.used + 2 <= pf.pool.size();
       if (prof) HIP_TRY(hipEventRecord(pf.pool[pf.used], stream));
       const int rc = (LY == 256 && LX == 256) ? launch_fft_xy256(xa, stream)
-                                               : launch_fft_plane(LY, LX, xa, stream, plan.split);
+                                               : launch_fft_plane(LY, LX, xa, stream, plan.split, plan.prec);
       if (prof) {
         HIP_TRY(hipEventRecord(pf.pool[pf.used + 1], stream));
         char lab[64];
-        snprintf(lab, sizeof(lab), "fft_plane_f32%s_%dx%d", plan.split ? "_split" : "", LY, LX);
+        snprintf(lab, sizeof(lab), "fft_plane_%s%s_%dx%d", plan.prec == PREC_F64 ? "f64" : "f32",
+                 plan.split ? "_split" : "", LY, LX);
         pf.recs.push_back({lab, pf.pool[pf.used], pf.pool[pf.used + 1]});
         pf.used += 2;
       }
@@ -845,6 +857,7 @@ static int run_plan(Plan& plan, const void* din, void* dout, bool inverse, hipSt
       ca.w_mask = (unsigned long long)plan.per - 1ULL;
       ca.inverse = inverse ? 1 : 0;
       ca.split = plan.split ? 1 : 0;
+      ca.f64 = plan.prec == PREC_F64 ? 1 : 0;
       Prof& pf = P();
       const bool prof = pf.on && !resolve && pf.used + 2 <= pf.pool.size();
       if (prof) HIP_TRY(hipEventRecord(pf.pool[pf.used], stream));
@@ -852,7 +865,8 @@ static int run_plan(Plan& plan, const void* din, void* dout, bool inverse, hipSt
       if (prof) {
         HIP_TRY(hipEventRecord(pf.pool[pf.used + 1], stream));
         char lab[64];
-        snprintf(lab, sizeof(lab), "fft_cube_%s_f32%s_%d", A ? "a" : "b", plan.split ? "_split" : "", ca.n);
+        snprintf(lab, sizeof(lab), "fft_cube_%s_%s%s_%d", A ? "a" : "b", ca.f64 ? "f64" : "f32",
+                 plan.split ? "_split" : "", ca.n);
         pf.recs.push_back({lab, pf.pool[pf.used], pf.pool[pf.used + 1]});
         pf.used += 2;
       }
@@ -1963,12 +1977,12 @@ int describe_plan(int rank, const size_t* dims, size_t batch, unsigned flags, in
                        d.mode == MODE_PLANE ? (d.K == 256 ? 64 : (long long)d.K)
                        : d.mode == MODE_COL4096 ? 16
                        : d.mode == MODE_CUBE_A ? (d.lg == 9 ? 64 : (1LL << d.lg) / 4)   // rows per workgroup
-                       : d.mode == MODE_CUBE_B ? (d.lg == 9 ? 8 : d.lg == 8 ? 16 : 32)   // columns per workgroup (x 8 or 4 rows x n planes)
+                       : d.mode == MODE_CUBE_B ? (d.lg == 9 ? 8 : d.lg == 8 || prec == PREC_F64 ? 16 : 32)   // columns per workgroup (x 8 or 4 rows x n planes)
                        : pass_cols(d, p.split, prec),
                        d.mode == MODE_PLANE ? plane_threads(d)
                        : d.mode == MODE_COL4096 ? 512
                        : d.mode == MODE_CUBE_A ? (d.lg == 9 ? 1024 : d.lg == 8 ? 512 : 256)
-                       : d.mode == MODE_CUBE_B ? (d.lg == 9 ? 1024 : 512)
+                       : d.mode == MODE_CUBE_B ? (d.lg == 9 ? 1024 : prec == PREC_F64 ? 256 : 512)
                        : pass_cols(d, p.split, prec) * geom_tpl(1 << d.lg)};
     for (int k = 0; k < NF; ++k) f[k] = v[k];
   }

@@ -254,6 +254,23 @@ __global__ void __launch_bounds__(C1B_NT, 4) k_fft_cube128_b(const CubeArgs a) {
   cube128_b_tile<INV, WS, SPLIT>(a, blockIdx.x, buf, atab, (int)threadIdx.x);
 }
 
+// FP64 128^3 blocks: pass A's 64 KiB tile with 256 threads of 16 points, pass
+// B's 128 KiB tile with 256 threads of 32, two workgroups per CU each.  HBM
+// bound: two passes instead of three line passes, 2 x 128^3 inverse 71.2 ->
+// 49.9 us, 4 x 128^3 134.6 -> 97.5 us (5.5 TB/s over the two passes).
+template <bool INV>
+__global__ void __launch_bounds__(C1_NT) k_fft_cube128d_a(const CubeArgs a) {
+  __shared__ cpx<double> buf[C1A_LDS];
+  __shared__ cpx<double> tws[C1A_TWS];
+  cube128_a_tile<INV, false, false, double>(a, blockIdx.x, buf, tws, (int)threadIdx.x);
+}
+
+template <bool INV>
+__global__ void __launch_bounds__(C1ZG<double>::NT) k_fft_cube128d_b(const CubeArgs a) {
+  __shared__ cpx<double> buf[C1ZG<double>::LDS_ELEMS];
+  cube128_b_tile<INV, false, false, double>(a, blockIdx.x, buf, nullptr, (int)threadIdx.x);
+}
+
 void preload_cube() { preload_kernel(reinterpret_cast<const void*>(&k_fft_cube_a<false, false, false>)); }
 
 static bool cube_grid(unsigned long long nplanes, unsigned long long per, unsigned long long* blocks) {
@@ -283,8 +300,14 @@ int launch_fft_cube_a(const CubeArgs& a, void* stream) {
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   unsigned long long blocks;
   if ((a.n != CB_L && a.n != C1_L) || a.nplanes == 0 || !cube_grid(a.nplanes, 4, &blocks) || a.w_store ||
-      (a.tab && (a.n != C1_L || a.w_load)) || (a.split && a.w_load))
+      (a.tab && (a.n != C1_L || a.w_load)) || (a.split && a.w_load) || (a.f64 && (a.n != C1_L || a.split || a.w_load)))
     return -1;
+  if (a.f64) {
+    const dim3 g((unsigned)blocks), t(C1_NT);
+    if (a.inverse) FFTAMD_LAUNCH((k_fft_cube128d_a<true>), g, t, 0, s, a);
+    else FFTAMD_LAUNCH((k_fft_cube128d_a<false>), g, t, 0, s, a);
+    return hipGetLastError() == hipSuccess ? 0 : -2;
+  }
   if (a.n == C1_L) {
     const dim3 g((unsigned)blocks), t(C1_NT);
     CUBE_DISPATCH(k_fft_cube128_a, a.w_load, g, t, s, a);
@@ -300,8 +323,15 @@ int launch_fft_cube_b(const CubeArgs& a, void* stream) {
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   unsigned long long blocks;
   if ((a.n != CB_L && a.n != C1_L) || a.nplanes == 0 || a.nplanes % a.n || a.w_load ||
-      (a.tab && (a.n != C1_L || a.w_store)) || (a.split && a.w_store))
+      (a.tab && (a.n != C1_L || a.w_store)) || (a.split && a.w_store) || (a.f64 && (a.n != C1_L || a.split || a.w_store)))
     return -1;
+  if (a.f64) {
+    if (!cube_grid(a.nplanes / C1_L, 32 * (C1_L / C1B_COLS<double>), &blocks)) return -1;
+    const dim3 g((unsigned)blocks), t(C1ZG<double>::NT);
+    if (a.inverse) FFTAMD_LAUNCH((k_fft_cube128d_b<true>), g, t, 0, s, a);
+    else FFTAMD_LAUNCH((k_fft_cube128d_b<false>), g, t, 0, s, a);
+    return hipGetLastError() == hipSuccess ? 0 : -2;
+  }
   if (a.n == C1_L) {
     if (!cube_grid(a.nplanes / C1_L, 128, &blocks)) return -1;
     const dim3 g((unsigned)blocks), t(C1B_NT);

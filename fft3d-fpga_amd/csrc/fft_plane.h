@@ -30,10 +30,12 @@ int launch_fft_xy256(const PlaneArgs& a, void* stream);
 
 // LY x LX planes with 16 <= LY, LX <= 128 and LY * LX >= 1024, one workgroup
 // per plane holding it in LDS (fft_plane.hip).  split: radix-16 stages on FP16
-// matrix cores with hi+lo operands.  0 on success, -1 for an unsupported
-// shape or grid, -2 on a launch error.  In place allowed.
-int launch_fft_plane(int ly, int lx, const PlaneArgs& a, void* stream, bool split = false);
-bool plane_shape_supported(long long ly, long long lx);
+// matrix cores with hi+lo operands.  FP64: up to PLANE_F64_MAX points, no
+// weights.  0 on success, -1 for an unsupported shape or grid, -2 on a launch
+// error.  In place allowed.
+constexpr long long PLANE_F64_MAX = 8192;
+int launch_fft_plane(int ly, int lx, const PlaneArgs& a, void* stream, bool split = false, int prec = 0);
+bool plane_shape_supported(long long ly, long long lx, int prec = 0);
 
 // The 4096-point transform along the second-fastest axis of blocks of 4096
 // rows of lx elements (fft_col.hip): element (o, row, x) at o * in_o + row *
@@ -75,13 +77,14 @@ struct CubeArgs {
   unsigned long long nplanes;    // n x n planes in the array (a multiple of n for pass B)
   const void* tw;                // Stockham twiddles of n-point lines (n = 512: of the
                                  // 64-point lines of pass A, the 128-point lines of pass B)
-  const void* w256;              // W256^m, m = 0..255
+  const void* w256;              // W256^m, m = 0..255 (in the values' precision)
   const void* w512;              // W512^m, m = 0..511 (n = 512)
   const float* w_load;
   const float* w_store;
   unsigned long long w_mask;
   int inverse;
   int split;                     // radix-16 stages on FP16 MFMA with hi + lo operands (no weights)
+  int f64;                       // FP64 values and tables (n = 128, no weights)
   // optional transform table (n = 128 only, no weights): block t starts at
   // tab[2 t] in `in` and tab[2 t + 1] in `out` (complex elements); NULL:
   // block t at t n^3 in both

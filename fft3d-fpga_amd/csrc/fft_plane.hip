@@ -24,10 +24,15 @@
 namespace fftamd {
 
 // SPLIT: radix-16 stages on FP16 matrix cores with hi+lo operands (fft_split.h).
-template <int LY, int LX, bool INV, bool SPLIT>
+// FP64 planes of up to 8192 points (139 KiB of LDS; up to 4096 points two
+// workgroups per CU): a 3D array of such planes takes two passes over HBM
+// instead of three line passes.  30 x 64^3 129.8 -> 92.4 us, 200 x 32^3 128.5
+// -> 78.6 us; 8192 points, one workgroup per CU: 500 planes of 64 x 128 46.6 ->
+// 30.5 us, 13 x (64 x 128 x 64) 117.7 -> 97.5 us.
+template <int LY, int LX, bool INV, bool SPLIT, typename R = float>
 __global__ void __launch_bounds__(LY * LX / 16) k_fft_plane(const PlaneArgs a) {
-  __shared__ cpx<float> lds[PlaneGeom<LY, LX, SPLIT>::LDS];
-  plane_tile<LY, LX, INV, SPLIT>(a, blockIdx.x, lds, (int)threadIdx.x);
+  __shared__ cpx<R> lds[PlaneGeom<LY, LX, SPLIT>::LDS];
+  plane_tile<LY, LX, INV, SPLIT, R>(a, blockIdx.x, lds, (int)threadIdx.x);
 }
 
 // The 128 x 128 plane (128 KiB) in two halves: 512 threads hold the plane in
@@ -134,13 +139,8 @@ static void launch_halves(const PlaneArgs& a, hipStream_t s) {
   }
 }
 
-bool plane_shape_supported(long long ly, long long lx) {
-  auto p2 = [](long long v) { return v >= 16 && v <= 128 && (v & (v - 1)) == 0; };
-  return p2(ly) && p2(lx) && ly * lx >= 1024;
-}
-
 template <int LY, int LX, bool SPLIT>
-static void launch_shape(const PlaneArgs& a, hipStream_t s) {
+static void launch_shape_f32(const PlaneArgs& a, hipStream_t s) {
   constexpr int NT = PlaneGeom<LY, LX, SPLIT>::NT;
   // two workgroups per CU (FP32 stages; split-precision stages would spill
   // registers at 512 threads and keep the whole-plane kernel)
@@ -155,36 +155,57 @@ static void launch_shape(const PlaneArgs& a, hipStream_t s) {
   }
 }
 
-template <int LY, bool SPLIT>
+bool plane_shape_supported(long long ly, long long lx, int prec) {
+  auto p2 = [](long long v) { return v >= 16 && v <= 128 && (v & (v - 1)) == 0; };
+  return p2(ly) && p2(lx) && ly * lx >= 1024 && (prec == PREC_F32 || ly * lx <= PLANE_F64_MAX);
+}
+
+template <int LY, int LX, bool SPLIT, typename R>
+static void launch_shape(const PlaneArgs& a, hipStream_t s) {
+  if constexpr (sizeof(R) == 8) {
+    if constexpr (LY * LX <= PLANE_F64_MAX) {
+      const dim3 g((unsigned)a.nplanes), t(PlaneGeom<LY, LX, false>::NT);
+      if (a.inverse) FFTAMD_LAUNCH((k_fft_plane<LY, LX, true, false, double>), g, t, 0, s, a);
+      else FFTAMD_LAUNCH((k_fft_plane<LY, LX, false, false, double>), g, t, 0, s, a);
+    }
+    return;
+  } else {
+    launch_shape_f32<LY, LX, SPLIT>(a, s);
+  }
+}
+
+template <int LY, bool SPLIT, typename R>
 static bool dispatch_lx(int lx, const PlaneArgs& a, hipStream_t s) {
   switch (lx) {
-    case 16: if constexpr (LY * 16 >= 1024) { launch_shape<LY, 16, SPLIT>(a, s); return true; } else return false;
-    case 32: if constexpr (LY * 32 >= 1024) { launch_shape<LY, 32, SPLIT>(a, s); return true; } else return false;
-    case 64: launch_shape<LY, 64, SPLIT>(a, s); return true;
-    case 128: launch_shape<LY, 128, SPLIT>(a, s); return true;
+    case 16: if constexpr (LY * 16 >= 1024) { launch_shape<LY, 16, SPLIT, R>(a, s); return true; } else return false;
+    case 32: if constexpr (LY * 32 >= 1024) { launch_shape<LY, 32, SPLIT, R>(a, s); return true; } else return false;
+    case 64: launch_shape<LY, 64, SPLIT, R>(a, s); return true;
+    case 128: launch_shape<LY, 128, SPLIT, R>(a, s); return true;
     default: return false;
   }
 }
 
-template <bool SPLIT>
+template <bool SPLIT, typename R = float>
 static bool dispatch_ly(int ly, int lx, const PlaneArgs& a, hipStream_t s) {
   switch (ly) {
-    case 16: return dispatch_lx<16, SPLIT>(lx, a, s);
-    case 32: return dispatch_lx<32, SPLIT>(lx, a, s);
-    case 64: return dispatch_lx<64, SPLIT>(lx, a, s);
-    case 128: return dispatch_lx<128, SPLIT>(lx, a, s);
+    case 16: return dispatch_lx<16, SPLIT, R>(lx, a, s);
+    case 32: return dispatch_lx<32, SPLIT, R>(lx, a, s);
+    case 64: return dispatch_lx<64, SPLIT, R>(lx, a, s);
+    case 128: return dispatch_lx<128, SPLIT, R>(lx, a, s);
     default: return false;
   }
 }
 
 void preload_plane() { preload_kernel(reinterpret_cast<const void*>(&k_fft_plane<64, 64, false, false>)); }
 
-int launch_fft_plane(int ly, int lx, const PlaneArgs& a, void* stream, bool split) {
+int launch_fft_plane(int ly, int lx, const PlaneArgs& a, void* stream, bool split, int prec) {
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  if (!plane_shape_supported(ly, lx) || a.nplanes == 0 || a.nplanes > 0xFFFFFFFFull / 1024 ||
+  if (!plane_shape_supported(ly, lx, prec) || (prec == PREC_F64 && (split || a.w_load || a.w_store)) || a.nplanes == 0 || a.nplanes > 0xFFFFFFFFull / 1024 ||
       (a.tab && a.ppt == 0))
     return -1;
-  const bool ok = split ? dispatch_ly<true>(ly, lx, a, s) : dispatch_ly<false>(ly, lx, a, s);
+  const bool ok = prec == PREC_F64 ? dispatch_ly<false, double>(ly, lx, a, s)
+                  : split           ? dispatch_ly<true>(ly, lx, a, s)
+                                    : dispatch_ly<false>(ly, lx, a, s);
   if (!ok) return -1;
   return hipGetLastError() == hipSuccess ? 0 : -2;
 }

@@ -24,8 +24,8 @@ struct PlaneGeom {
 // threads tid = 0 .. NT - 1 with PlaneGeom::LDS elements of LDS at lds.
 // SPLIT: radix-16 stages on FP16 matrix cores with hi+lo operands
 // (fft_split.h; a tile is then made of whole waves).
-template <int LY, int LX, bool INV, bool SPLIT>
-__device__ __forceinline__ void plane_tile(const PlaneArgs& a, unsigned long long plane, cpx<float>* lds,
+template <int LY, int LX, bool INV, bool SPLIT, typename R = float>
+__device__ __forceinline__ void plane_tile(const PlaneArgs& a, unsigned long long plane, cpx<R>* lds,
                                            int tid) {
   using PG = PlaneGeom<LY, LX, SPLIT>;
   using GX = typename PG::GX;
@@ -36,9 +36,9 @@ __device__ __forceinline__ void plane_tile(const PlaneArgs& a, unsigned long lon
     base = (long long)a.tab[2 * t] + (long long)z * (LY * LX);
     obase = (long long)a.tab[2 * t + 1] + (long long)z * (LY * LX);
   }
-  const cpx<float>* __restrict__ in = reinterpret_cast<const cpx<float>*>(a.in) + base;
-  cpx<float>* __restrict__ out = reinterpret_cast<cpx<float>*>(a.out) + obase;
-  cpx<float> v[16];
+  const cpx<R>* __restrict__ in = reinterpret_cast<const cpx<R>*>(a.in) + base;
+  cpx<R>* __restrict__ out = reinterpret_cast<cpx<R>*>(a.out) + obase;
+  cpx<R> v[16];
 
   // ---- rows: thread (row c, tau); stage 0 reads its butterfly inputs from HBM
   {
@@ -50,13 +50,12 @@ __device__ __forceinline__ void plane_tile(const PlaneArgs& a, unsigned long lon
 #pragma unroll
       for (int r = 0; r < RAD; ++r) {
         const int e = c * LX + j + r * (LX / RAD);
-        cpx<float> x = in[e];
-        if (a.w_load) x = cscale(x, a.w_load[(unsigned long long)(base + e) & a.w_mask]);
+        cpx<R> x = in[e];
+        if (a.w_load) x = cscale(x, (R)a.w_load[(unsigned long long)(base + e) & a.w_mask]);
         v[b * RAD + r] = INV ? cswap(x) : x;
       }
     }
-    run_stages<float, LX, MODE_CONTIG, 0, SPLIT, LY>(v, lds, c, tau,
-                                                     reinterpret_cast<const cpx<float>*>(a.tw_x));
+    run_stages<R, LX, MODE_CONTIG, 0, SPLIT, LY>(v, lds, c, tau, reinterpret_cast<const cpx<R>*>(a.tw_x));
     // last stage: point k = j + r*NS of row c -> column layout
     constexpr int NPX = GX::NP;
     constexpr int RL = sched_radix(LX, NPX - 1), NSL = sched_ns(LX, NPX - 1), NBL = 16 / RL;
@@ -73,10 +72,9 @@ __device__ __forceinline__ void plane_tile(const PlaneArgs& a, unsigned long lon
   // ---- columns: thread (column c, tau), adjacent threads on adjacent columns
   {
     const int c = tid % LX, tau = tid / LX;
-    stage_load_lds<float, LY, MODE_STRIDED, 0, LX>(v, lds, c, tau);
+    stage_load_lds<R, LY, MODE_STRIDED, 0, LX>(v, lds, c, tau);
     __syncthreads();  // every thread holds its stage-0 inputs before stage 0 stores
-    run_stages<float, LY, MODE_STRIDED, 0, SPLIT, LX>(v, lds, c, tau,
-                                                      reinterpret_cast<const cpx<float>*>(a.tw_y));
+    run_stages<R, LY, MODE_STRIDED, 0, SPLIT, LX>(v, lds, c, tau, reinterpret_cast<const cpx<R>*>(a.tw_y));
     constexpr int NPY = GY::NP;
     constexpr int RL = sched_radix(LY, NPY - 1), NSL = sched_ns(LY, NPY - 1), NBL = 16 / RL;
 #pragma unroll
@@ -85,9 +83,9 @@ __device__ __forceinline__ void plane_tile(const PlaneArgs& a, unsigned long lon
 #pragma unroll
       for (int r = 0; r < RL; ++r) {
         const int e = (j + r * NSL) * LX + c;
-        cpx<float> x = v[b * RL + r];
+        cpx<R> x = v[b * RL + r];
         if (INV) x = cswap(x);
-        if (a.w_store) x = cscale(x, a.w_store[(unsigned long long)(obase + e) & a.w_mask]);
+        if (a.w_store) x = cscale(x, (R)a.w_store[(unsigned long long)(obase + e) & a.w_mask]);
         out[e] = x;
       }
     }

@@ -214,5 +214,11 @@ __device__ __forceinline__ void wg_dft16(cpx<float>* v, const split_half8* atab 
     dft16(v);
   }
 }
+// the same for either precision (FP64 has no split form)
+template <bool SPLIT, bool TAB, typename R>
+__device__ __forceinline__ void wg_dft16_r(cpx<R>* v, const split_half8* atab = nullptr) {
+  if constexpr (sizeof(R) == 4) wg_dft16<SPLIT, TAB>(v, atab);
+  else dft16(v);
+}
 
 }  // namespace fftamd
