@@ -58,6 +58,11 @@ int dev_c2c_noalloc(int rank, const size_t* dims, size_t batch, const void* din,
 int dev_c2c_weighted(int rank, const size_t* dims, size_t batch, const void* din, void* dout,
                      bool inverse, const float* w_load, const float* w_store, void* stream);
 
+// gw = sum over the batch of Re(conj(g) fx), FP32: the gradient of the weights
+// of w . F(x) for the upstream gradient g and fx = F(x).
+int dev_weight_grad(int rank, const size_t* dims, size_t batch, const void* g, const void* fx, void* gw,
+                    void* stream);
+
 // ---- multi-transform plans (uneven sizes, one persistent launch) ---------------
 int multi_create(void** handle, unsigned count, const unsigned* dims3, const unsigned long long* in_off,
                  const unsigned long long* out_off, const void* din, void* dout, bool inverse,

@@ -1854,6 +1854,7 @@ int runtime_init(int dev, bool svm) {
   preload_plane();
   preload_multi();
   preload_flow();
+  preload_wgrad();
   st.dev = dev;
   st.svm = svm;
   st.ready = true;
@@ -2240,6 +2241,33 @@ static int check_dev_buffers(int rank, const size_t* dims, size_t batch, const v
   const uintptr_t a = reinterpret_cast<uintptr_t>(din), b = reinterpret_cast<uintptr_t>(dout);
   if (a != b && a < b + bytes && b < a + bytes) {
     set_error("input and output buffers overlap without being the same buffer (in place needs d_in == d_out)");
+    return -1;
+  }
+  return 0;
+}
+
+int dev_weight_grad(int rank, const size_t* dims, size_t batch, const void* g, const void* fx, void* gw,
+                    void* stream) {
+  if (!check_dims(rank, dims, batch)) return -1;
+  size_t points = 1;
+  for (int d = 0; d < rank; ++d) points *= dims[d];
+  if (!gw || check_dev_buffers(rank, dims, batch, g, fx, 8)) {
+    if (!gw) set_error("null device pointer");
+    return -1;
+  }
+  const uintptr_t w0 = reinterpret_cast<uintptr_t>(gw), w1 = w0 + 4 * points;
+  for (const void* p : {g, fx}) {
+    const uintptr_t a = reinterpret_cast<uintptr_t>(p);
+    if (w0 < a + 8 * points * batch && a < w1) {
+      set_error("the weight gradient overlaps an input");
+      return -1;
+    }
+  }
+  State& st = S();
+  std::lock_guard<std::recursive_mutex> lk(st.mu);
+  if (runtime_ensure_device()) return -1;
+  if (launch_weight_grad(g, fx, gw, points, (unsigned)batch, stream)) {
+    set_error("weight gradient launch failed: %s", hipGetErrorString(hipGetLastError()));
     return -1;
   }
   return 0;

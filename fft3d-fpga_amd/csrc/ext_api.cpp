@@ -55,6 +55,13 @@ int fftamd_c2c_weighted_dev(int rank, const unsigned* dims, unsigned batch, cons
   return fftamd::dev_c2c_weighted(rank, d, batch, d_in, d_out, inverse != 0, w_in, w_out, stream);
 }
 
+int fftamd_weight_grad_dev(int rank, const unsigned* dims, unsigned batch, const float2* d_g,
+                           const float2* d_fx, float* d_gw, void* stream) {
+  size_t d[3];
+  if (!dims_ok(rank, dims, batch, d)) return -1;
+  return fftamd::dev_weight_grad(rank, d, batch, d_g, d_fx, d_gw, stream);
+}
+
 int fftfpgaf_c2c_3d_ddr_dev(unsigned N, const float2* d_in, float2* d_out, bool inv,
                             unsigned how_many, void* stream) {
   if (d_in == nullptr || d_out == nullptr || N == 0 || (N & (N - 1)) != 0 || how_many == 0) {

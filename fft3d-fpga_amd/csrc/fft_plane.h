@@ -95,4 +95,10 @@ int launch_fft_cube_b(const CubeArgs& a, void* stream);
 int launch_fft_c512_a(const CubeArgs& a, void* stream);  // n = 512 (fft_cube512.hip)
 int launch_fft_c512_b(const CubeArgs& a, void* stream);
 
+// gw[i] = sum_b Re(conj(g[b][i]) f[b][i]) for FP32 complex g, f of batch x
+// points values (fft_wgrad.hip).  0 on success, -1 when the grid does not fit,
+// -2 on a launch error.
+int launch_weight_grad(const void* g, const void* f, void* gw, unsigned long long points, unsigned batch,
+                       void* stream);
+
 }  // namespace fftamd

@@ -25,6 +25,7 @@ void preload_col();
 void preload_plane();
 void preload_multi();
 void preload_flow();
+void preload_wgrad();
 inline void preload_kernel(const void* f) {
   hipFuncAttributes fa;
   (void)hipFuncGetAttributes(&fa, f);

@@ -71,6 +71,7 @@ SIGNATURES = {
     "fftamd_c2c_dev_noalloc": (_i, [_i, ctypes.POINTER(_u), _u, _vp, _vp, _i, _u, _vp]),
     "fftamd_z2z_dev": (_i, [_i, ctypes.POINTER(_u), _u, _vp, _vp, _i, _u, _vp]),
     "fftamd_c2c_weighted_dev": (_i, [_i, ctypes.POINTER(_u), _u, _vp, _vp, _i, _vp, _vp, _vp]),
+    "fftamd_weight_grad_dev": (_i, [_i, ctypes.POINTER(_u), _u, _vp, _vp, _vp, _vp]),
     "fftfpgaf_c2c_3d_ddr_dev": (_i, [_u, _vp, _vp, _b, _u, _vp]),
     "fftamd_multi_create": (_i, [ctypes.POINTER(_vp), _u, _vp, _vp, _vp, _i, _u]),
     "fftamd_multi_exec": (_i, [_vp, _vp]),

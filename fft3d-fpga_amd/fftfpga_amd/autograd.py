@@ -15,6 +15,7 @@ inputs is followed (grad = 2 dL/d conj(x) for a real loss).  A gradient for
 from __future__ import annotations
 
 import ctypes
+import math
 
 import torch
 
@@ -58,6 +59,26 @@ def weighted_transform(x, rank, inverse=False, w_in=None, w_out=None, out=None):
     return out
 
 
+def weight_gradient(g, fx, rank):
+    """Re sum over the batch of conj(g) . fx, one float per point of a transform (no autograd)."""
+    _check(fx, rank)
+    dims = [int(d) for d in fx.shape[fx.dim() - rank:]]
+    # a lazily conjugated or negated gradient is made plain: the kernel reads its memory
+    g, fx = g.resolve_conj().resolve_neg().contiguous(), fx.contiguous()
+    if g.dtype != fx.dtype or g.shape != fx.shape or g.device != fx.device:
+        raise ValueError("g must match fx")
+    points = math.prod(dims)
+    if fx.numel() == 0:
+        return torch.zeros(dims, dtype=torch.float32, device=fx.device)
+    gw = torch.empty(dims, dtype=torch.float32, device=fx.device)
+    cd = (ctypes.c_uint * rank)(*dims)
+    rc = load().fftamd_weight_grad_dev(rank, cd, fx.numel() // points, ctypes.c_void_p(g.data_ptr()),
+                                       ctypes.c_void_p(fx.data_ptr()), ctypes.c_void_p(gw.data_ptr()), _stream(fx))
+    if rc != 0:
+        raise RuntimeError(f"fftamd weight gradient failed: {last_error()}")
+    return gw
+
+
 class _WeightedFFT(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, weight, rank, inverse):
@@ -86,8 +107,11 @@ class _WeightedFFT(torch.autograd.Function):
         gw = None
         if ctx.has_w and ctx.needs_input_grad[1]:
             fx = weighted_transform(x, ctx.rank, inverse=ctx.inverse)
-            prod = (torch.conj(g) * fx).real
-            gw = prod.reshape(-1, *w.shape).sum(0)
+            if torch.is_grad_enabled():  # create_graph: torch records the product
+                prod = (torch.conj(g) * fx).real
+                gw = prod.reshape(-1, *w.shape).sum(0)
+            else:
+                gw = weight_gradient(g, fx, ctx.rank)
         return gx, gw, None, None
 
 

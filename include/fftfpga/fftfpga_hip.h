@@ -101,6 +101,13 @@ int fftamd_c2c_weighted_dev(int rank, const unsigned *dims, unsigned batch, cons
                             float2 *d_out, int inverse, const float *w_in, const float *w_out,
                             void *stream);
 
+/* Gradient of the weights of w_out .* F(in): d_gw[i] = sum over the batch of
+ * Re(conj(d_g) d_fx)[i] for the upstream gradient d_g and the unweighted
+ * transform d_fx = F(in), both `batch` contiguous transforms; d_gw holds one
+ * transform's points.  One pass over both inputs, summed in FP64. */
+int fftamd_weight_grad_dev(int rank, const unsigned *dims, unsigned batch, const float2 *d_g,
+                           const float2 *d_fx, float *d_gw, void *stream);
+
 /* Device-pointer twin of fftfpgaf_c2c_3d_ddr / _3d_ddr_batch: how_many
  * contiguous N^3 transforms (how_many >= 1). */
 int fftfpgaf_c2c_3d_ddr_dev(unsigned N, const float2 *d_in, float2 *d_out, bool inv,
