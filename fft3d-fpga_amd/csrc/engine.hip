@@ -397,13 +397,23 @@ static int split_strided(int prec, int lg, int* lg1, int* lg2) {
   return 0;
 }
 
-// Fewest planes for which a plane pass replaces the separate x and y passes:
-// any count for planes up to 128 x 128 (one workgroup per plane, measured
-// faster from one 64 x 64 plane up); 32 for 256 x 256 planes (four workgroups
+// Fewest planes for which a plane pass replaces the separate x and y passes
+// (one workgroup per plane).  Any count for planes up to 128 x 128 (measured
+// faster from one 64 x 64 plane up) and of up to 4096 points (one 256 x 16
+// plane 5.7 against 7.4 us); with a longer side 16 at 8192 points (8 planes of
+// 512 x 16 9.2 against 8.7 us, 64 10.0 against 13.6; of 32 x 256 6.4 against 7.8
+// and 7.1 against 10.0), 128 at 16384 (64 planes of 32 x 512 14.5 against 12.5
+// us, 128 16.0 against 17.8; of 64 x 256 12.3 against 12.5 and 13.3 against 17.9)
+// and 256 at 32768 (128 planes of 64 x 512 28.5 against 25.6 us, 256 43.2 against
+// 53.5; of 128 x 256 22.7 against 24.7 and 32.9 against 52.7).  32 for 256 x 256 planes (four workgroups
 // per plane; with 16 or fewer planes the x and y line passes are faster,
 // measured 13.9 against 16.9 us at 16 planes, 20.6 against 18.1 at 32).
 static constexpr unsigned long long PLANE_MIN_COUNT = 1;
 static constexpr unsigned long long PLANE256_MIN_COUNT = 32;
+static constexpr unsigned long long plane_min_count(long long ly, long long lx) {
+  if (ly <= 128 && lx <= 128) return PLANE_MIN_COUNT;
+  return ly * lx <= 4096 ? 1 : ly * lx <= 8192 ? 16 : ly * lx <= 16384 ? 128 : 256;
+}
 // most planes of one launch (grid size in work-items is 32-bit)
 static constexpr unsigned long long PLANE_MAX_COUNT = 0xFFFFFFFFull / 1024;
 // Fewest 16-column groups for which the one-pass 4096-point column transform
@@ -494,7 +504,8 @@ static int build_plan(int rank, const size_t* dims, size_t batch, unsigned flags
     for (int d = 0; d < rank - 2; ++d) O *= dims[d];
     const bool big = prec == PREC_F32 && LY == 256 && LX == 256;  // no split-precision variant
     if ((big && !plan.split && O >= PLANE256_MIN_COUNT) ||
-        (plane_shape_supported(LY, LX, prec) && O >= PLANE_MIN_COUNT && (prec == PREC_F32 || O <= PLANE_MAX_COUNT))) {
+        (plane_shape_supported(LY, LX, pass_kind(plan.split, prec)) && O >= plane_min_count(LY, LX) &&
+         (O <= PLANE_MAX_COUNT || (prec == PREC_F32 && LY <= 128 && LX <= 128)))) {
       PassDesc p;
       p.lg = ilog2c(LX);
       p.mode = MODE_PLANE;
@@ -993,6 +1004,11 @@ struct PlaneGroup {
   bool cube = false;            // 128^3 transforms whose input and output do not overlap: the y-split pair
 };
 
+// planes that the grouped launches of an uneven batch take
+static bool multi_plane_shape(long long ly, long long lx) {
+  return ly <= 128 && lx <= 128 && plane_shape_supported(ly, lx, KIND_F32);
+}
+
 struct MultiPlan {
   std::vector<MultiPass> passes;
   std::vector<MultiItem> items;
@@ -1334,7 +1350,7 @@ int multi_create(void** handle, unsigned count, const unsigned* dims3, const uns
   mp->inverse = inverse;
   mp->plane_ok = nphase == 3;
   for (unsigned i = 0; i < count && mp->plane_ok; ++i)
-    mp->plane_ok = trs[i].ps.size() == 3 && plane_shape_supported(dims3[3 * i + 1], dims3[3 * i + 2]);
+    mp->plane_ok = trs[i].ps.size() == 3 && multi_plane_shape(dims3[3 * i + 1], dims3[3 * i + 2]);
   if (mp->plane_ok) {
     std::map<std::tuple<unsigned, unsigned, unsigned>, std::vector<unsigned>> by_shape;
     for (unsigned oi = 0; oi < count; ++oi) {
@@ -1964,10 +1980,11 @@ int describe_plan(int rank, const size_t* dims, size_t batch, unsigned flags, in
     return -1;
   }
   // threads per workgroup of a plane pass: 512 for 256 x 256 (four per plane)
-  // and for FP32 128 x 128 (two halves), LY * LX / 16 otherwise
+  // and half as many as points per 16 for FP32 planes in two halves
   auto plane_threads = [&](const PassDesc& d) -> long long {
-    if (d.K == 256 || (d.K == 128 && d.lg == 7 && !p.split)) return 512;
-    return ((long long)d.K << d.lg) / 16;
+    if (d.K == 256 && d.lg == 8) return 512;
+    const long long points = (long long)d.K << d.lg;
+    return points >= 16384 && !p.split ? points / 32 : points / 16;
   };
   for (int i = 0; i < n; ++i) {
     const PassDesc& d = p.passes[i];
@@ -1975,7 +1992,7 @@ int describe_plan(int rank, const size_t* dims, size_t batch, unsigned flags, in
     long long v[NF] = {d.lg, d.mode, d.epi, d.transposing, d.in_p, d.out_p, d.in_c, d.out_c,
                        d.in_k, d.out_k, d.in_o, d.out_o, d.ncol, d.K, d.kbits,
                        (long long)d.nouter, d.M, d.cshift, d.src, d.dst,
-                       d.mode == MODE_PLANE ? (d.K == 256 ? 64 : (long long)d.K)
+                       d.mode == MODE_PLANE ? (d.K == 256 && d.lg == 8 ? 64 : (long long)d.K)
                        : d.mode == MODE_COL4096 ? 16
                        : d.mode == MODE_CUBE_A ? (d.lg == 9 ? 64 : (1LL << d.lg) / 4)   // rows per workgroup
                        : d.mode == MODE_CUBE_B ? (d.lg == 9 ? 8 : d.lg == 8 || prec == PREC_F64 ? 16 : 32)   // columns per workgroup (x 8 or 4 rows x n planes)

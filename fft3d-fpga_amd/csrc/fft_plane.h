@@ -28,14 +28,13 @@ struct PlaneArgs {
 // and out must not overlap.
 int launch_fft_xy256(const PlaneArgs& a, void* stream);
 
-// LY x LX planes with 16 <= LY, LX <= 128 and LY * LX >= 1024, one workgroup
-// per plane holding it in LDS (fft_plane.hip).  split: radix-16 stages on FP16
-// matrix cores with hi+lo operands.  FP64: up to PLANE_F64_MAX points, no
-// weights.  0 on success, -1 for an unsupported shape or grid, -2 on a launch
+// LY x LX planes with 16 <= LY, LX <= 512 and 1024 <= LY * LX <= the kind's
+// maximum below, one workgroup per plane (fft_plane.hip).  split: radix-16
+// stages on FP16 matrix cores with hi+lo operands.  FP64: no weights.  0 on success, -1 for an unsupported shape or grid, -2 on a launch
 // error.  In place allowed.
-constexpr long long PLANE_F64_MAX = 8192;
+constexpr long long PLANE_F32_MAX = 32768, PLANE_SPLIT_MAX = 16384, PLANE_F64_MAX = 8192;
 int launch_fft_plane(int ly, int lx, const PlaneArgs& a, void* stream, bool split = false, int prec = 0);
-bool plane_shape_supported(long long ly, long long lx, int prec = 0);
+bool plane_shape_supported(long long ly, long long lx, int kind);  // kind: PassKind
 
 // The 4096-point transform along the second-fastest axis of blocks of 4096
 // rows of lx elements (fft_col.hip): element (o, row, x) at o * in_o + row *

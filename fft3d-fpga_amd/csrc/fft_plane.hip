@@ -1,5 +1,6 @@
 // fft_plane.hip -- the 2D transform of every LY x LX plane of an array in one
-// pass over HBM, for planes that fit one workgroup's LDS (LY, LX <= 128).
+// pass over HBM, for planes of 1024 to 32768 points with sides 16 to 512: up to
+// 8192 points the plane sits in one workgroup's LDS, above that in its registers.
 //
 // One workgroup per plane, LY * LX / 16 threads, 16 points per thread in both
 // phases.  Rows: each thread loads its first-stage butterfly inputs of one row
@@ -11,8 +12,13 @@
 // HBM instead of three, and the plane is read and written exactly once.
 //
 // The radix stages are the line passes' (fft_pass_dev.h), instantiated with a
-// whole plane's rows or columns per workgroup.  128 x 128 FP32 planes use
-// k_fft_plane_halves below (two workgroups per CU).
+// whole plane's rows or columns per workgroup.  FP32 planes of 16384 points and
+// more use k_fft_plane_halves below.
+//
+// HBM bound: one read and one write instead of the two of separate x and y line
+// passes.  1024 planes of 16 x 256 24.1 -> 12.8 us, of 512 x 16 103.6 -> 48.0, of
+// 32 x 256 52.7 -> 31.6, of 64 x 256 96.2 -> 60.5, of 512 x 32 133.0 -> 67.6; of 128 x
+// 256 (one workgroup per CU, 256 KiB planes) 197.4 -> 129.5.
 #include <hip/hip_runtime.h>
 
 #include "launch.h"
@@ -35,68 +41,69 @@ __global__ void __launch_bounds__(LY * LX / 16) k_fft_plane(const PlaneArgs a) {
   plane_tile<LY, LX, INV, SPLIT, R>(a, blockIdx.x, lds, (int)threadIdx.x);
 }
 
-// The 128 x 128 plane (128 KiB) in two halves: 512 threads hold the plane in
-// registers, 32 points each, and LDS stages half of it at a time (rows 0..63,
-// then 64..127; then columns 0..63, then 64..127).  LDS is then 68 KiB, so
-// two workgroups share a CU and one loads or stores while the other
-// computes; the whole-plane kernel above needs 136 KiB and runs one
-// workgroup per CU.
-template <int L, bool SPLIT>
+// Planes of 16384 points (128 KiB) and 32768 points (256 KiB) in two halves:
+// 512 or 1024 threads hold the plane in registers (32 points each) and LDS
+// stages half of it at a time (rows 0..LY/2-1, then the others; then columns
+// 0..LX/2-1, then the others).  At 16384 points LDS is then 68 KiB, so two
+// workgroups share a CU and one loads or stores while the other computes; the
+// whole-plane kernel above needs 136 KiB and runs one workgroup per CU.  At 32768
+// points (1024 threads, at most 139 KiB) it is one workgroup per CU.
+template <int LY, int LX>
 struct HalfGeom {
-  using GX = Geom<L, MODE_CONTIG, L / 2>;  // rows: L/2 lines of L points
-  using GY = Geom<L, MODE_STRIDED, L / 2>; // columns: L/2 lines of L points
-  static constexpr int NT = L * L / 32;
+  using GX = Geom<LX, MODE_CONTIG, LY / 2>;   // rows: LY/2 lines of LX points
+  using GY = Geom<LY, MODE_STRIDED, LX / 2>;  // columns: LX/2 lines of LY points
+  static constexpr int NT = LY * LX / 32;
   static_assert(GX::NT == NT && GY::NT == NT, "16 points per thread per half");
   static constexpr int LDS = GX::LDS_ELEMS > GY::LDS_ELEMS ? GX::LDS_ELEMS : GY::LDS_ELEMS;
   // last row stage: radix 16, one butterfly per thread, so point k = tau + TPL r
-  static_assert(sched_radix(L, GX::NP - 1) == 16 && sched_ns(L, GX::NP - 1) == GX::TPL,
-                "points tau + TPL r: r < 8 are columns 0 .. L/2 - 1");
+  static_assert(sched_radix(LX, GX::NP - 1) == 16 && sched_ns(LX, GX::NP - 1) == GX::TPL,
+                "points tau + TPL r: r < 8 are columns 0 .. LX/2 - 1");
 };
 
 // WL, WS: the launch carries load or store weights.
-template <int L, bool INV, bool SPLIT, bool WL, bool WS>
-__global__ void __launch_bounds__(L * L / 32, 4) k_fft_plane_halves(const PlaneArgs a) {
-  using HG = HalfGeom<L, SPLIT>;
+template <int LY, int LX, bool INV, bool WL, bool WS>
+__global__ void __launch_bounds__(LY * LX / 32, 4) k_fft_plane_halves(const PlaneArgs a) {
+  using HG = HalfGeom<LY, LX>;
   using GX = typename HG::GX;
   using GY = typename HG::GY;
-  constexpr int H = L / 2;
+  constexpr int HY = LY / 2, HX = LX / 2;
   __shared__ cpx<float> lds[HG::LDS];
   const unsigned long long plane = blockIdx.x;
   long long base = (long long)plane * a.plane_stride, obase = base;
   if (a.tab) {  // planes of a batch of transforms placed anywhere
     const unsigned t = (unsigned)(plane / a.ppt), z = (unsigned)(plane % a.ppt);
-    base = (long long)a.tab[2 * t] + (long long)z * (L * L);
-    obase = (long long)a.tab[2 * t + 1] + (long long)z * (L * L);
+    base = (long long)a.tab[2 * t] + (long long)z * (LY * LX);
+    obase = (long long)a.tab[2 * t + 1] + (long long)z * (LY * LX);
   }
   const cpx<float>* __restrict__ in = reinterpret_cast<const cpx<float>*>(a.in) + base;
   cpx<float>* __restrict__ out = reinterpret_cast<cpx<float>*>(a.out) + obase;
   const int tid = threadIdx.x;
-  cpx<float> rr[2][16];  // row results of row halves 0 and 1: point tau + TPL r of row c + H h
+  cpx<float> rr[2][16];  // row results of row halves 0 and 1: point tau + TPL r of row c + HY h
 
   // ---- rows, in two halves: thread (row c, tau); stage 0 reads from HBM
   const int rc = tid / GX::TPL, rtau = tid % GX::TPL;
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
-    constexpr int RAD = sched_radix(L, 0), NB = 16 / RAD;
+    constexpr int RAD = sched_radix(LX, 0), NB = 16 / RAD;
     cpx<float>* v = rr[h];
-    const int row = rc + H * h;
+    const int row = rc + HY * h;
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
       const int j = rtau + b * GX::TPL;
 #pragma unroll
       for (int r = 0; r < RAD; ++r) {
-        const int e = row * L + j + r * (L / RAD);
+        const int e = row * LX + j + r * (LX / RAD);
         cpx<float> x = in[e];
         if (WL) x = cscale(x, a.w_load[(unsigned long long)(base + e) & a.w_mask]);
         v[b * RAD + r] = INV ? cswap(x) : x;
       }
     }
     if (h) __syncthreads();  // the first half's last stage has read the buffer
-    run_stages<float, L, MODE_CONTIG, 0, SPLIT, H>(v, lds, rc, rtau, reinterpret_cast<const cpx<float>*>(a.tw_x));
+    run_stages<float, LX, MODE_CONTIG, 0, false, HY>(v, lds, rc, rtau, reinterpret_cast<const cpx<float>*>(a.tw_x));
   }
 
   // ---- columns, in two halves: thread (column c, tau), adjacent threads on adjacent columns
-  const int cc = tid % H, ctau = tid / H;
+  const int cc = tid % HX, ctau = tid / HX;
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
     __syncthreads();  // the previous stage has read the buffer
@@ -104,20 +111,20 @@ __global__ void __launch_bounds__(L * L / 32, 4) k_fft_plane_halves(const PlaneA
 #pragma unroll
     for (int rh = 0; rh < 2; ++rh)
 #pragma unroll
-      for (int r = 0; r < 8; ++r) lds[GY::idx(rtau + GX::TPL * r, rc + H * rh)] = rr[rh][8 * h + r];
+      for (int r = 0; r < 8; ++r) lds[GY::idx(rtau + GX::TPL * r, rc + HY * rh)] = rr[rh][8 * h + r];
     __syncthreads();
     cpx<float> v[16];
-    stage_load_lds<float, L, MODE_STRIDED, 0, H>(v, lds, cc, ctau);
+    stage_load_lds<float, LY, MODE_STRIDED, 0, HX>(v, lds, cc, ctau);
     __syncthreads();  // every thread holds its stage-0 inputs before stage 0 stores
-    run_stages<float, L, MODE_STRIDED, 0, SPLIT, H>(v, lds, cc, ctau, reinterpret_cast<const cpx<float>*>(a.tw_y));
+    run_stages<float, LY, MODE_STRIDED, 0, false, HX>(v, lds, cc, ctau, reinterpret_cast<const cpx<float>*>(a.tw_y));
     constexpr int NPY = GY::NP;
-    constexpr int RL = sched_radix(L, NPY - 1), NSL = sched_ns(L, NPY - 1), NBL = 16 / RL;
+    constexpr int RL = sched_radix(LY, NPY - 1), NSL = sched_ns(LY, NPY - 1), NBL = 16 / RL;
 #pragma unroll
     for (int b = 0; b < NBL; ++b) {
       const int j = ctau + b * GY::TPL;
 #pragma unroll
       for (int r = 0; r < RL; ++r) {
-        const int e = (j + r * NSL) * L + H * h + cc;
+        const int e = (j + r * NSL) * LX + HX * h + cc;
         cpx<float> x = v[b * RL + r];
         if (INV) x = cswap(x);
         if (WS) x = cscale(x, a.w_store[(unsigned long long)(obase + e) & a.w_mask]);
@@ -127,27 +134,27 @@ __global__ void __launch_bounds__(L * L / 32, 4) k_fft_plane_halves(const PlaneA
   }
 }
 
-template <int L, bool INV, bool SPLIT>
+template <int LY, int LX, bool INV>
 static void launch_halves(const PlaneArgs& a, hipStream_t s) {
-  const dim3 grid((unsigned)a.nplanes), block(HalfGeom<L, SPLIT>::NT);
+  const dim3 grid((unsigned)a.nplanes), block(HalfGeom<LY, LX>::NT);
   if (a.w_load) {
-    if (a.w_store) FFTAMD_LAUNCH((k_fft_plane_halves<L, INV, SPLIT, true, true>), grid, block, 0, s, a);
-    else FFTAMD_LAUNCH((k_fft_plane_halves<L, INV, SPLIT, true, false>), grid, block, 0, s, a);
+    if (a.w_store) FFTAMD_LAUNCH((k_fft_plane_halves<LY, LX, INV, true, true>), grid, block, 0, s, a);
+    else FFTAMD_LAUNCH((k_fft_plane_halves<LY, LX, INV, true, false>), grid, block, 0, s, a);
   } else {
-    if (a.w_store) FFTAMD_LAUNCH((k_fft_plane_halves<L, INV, SPLIT, false, true>), grid, block, 0, s, a);
-    else FFTAMD_LAUNCH((k_fft_plane_halves<L, INV, SPLIT, false, false>), grid, block, 0, s, a);
+    if (a.w_store) FFTAMD_LAUNCH((k_fft_plane_halves<LY, LX, INV, false, true>), grid, block, 0, s, a);
+    else FFTAMD_LAUNCH((k_fft_plane_halves<LY, LX, INV, false, false>), grid, block, 0, s, a);
   }
 }
 
 template <int LY, int LX, bool SPLIT>
 static void launch_shape_f32(const PlaneArgs& a, hipStream_t s) {
-  constexpr int NT = PlaneGeom<LY, LX, SPLIT>::NT;
-  // two workgroups per CU (FP32 stages; split-precision stages would spill
-  // registers at 512 threads and keep the whole-plane kernel)
-  if constexpr (LY == 128 && LX == 128 && !SPLIT) {
-    if (a.inverse) launch_halves<128, true, SPLIT>(a, s);
-    else launch_halves<128, false, SPLIT>(a, s);
+  if constexpr (LY * LX >= 16384 && !SPLIT) {
+    if (a.inverse) launch_halves<LY, LX, true>(a, s);
+    else launch_halves<LY, LX, false>(a, s);
   } else {
+    // split-precision stages would spill registers in the halves kernel and
+    // keep the whole plane in LDS (up to 16384 points)
+    constexpr int NT = PlaneGeom<LY, LX, SPLIT>::NT;
     if (a.inverse)
       FFTAMD_LAUNCH((k_fft_plane<LY, LX, true, SPLIT>), dim3((unsigned)a.nplanes), dim3(NT), 0, s, a);
     else
@@ -155,32 +162,38 @@ static void launch_shape_f32(const PlaneArgs& a, hipStream_t s) {
   }
 }
 
-bool plane_shape_supported(long long ly, long long lx, int prec) {
-  auto p2 = [](long long v) { return v >= 16 && v <= 128 && (v & (v - 1)) == 0; };
-  return p2(ly) && p2(lx) && ly * lx >= 1024 && (prec == PREC_F32 || ly * lx <= PLANE_F64_MAX);
+constexpr bool plane_shape_ok(long long ly, long long lx, int kind) {
+  return ly >= 16 && ly <= 512 && lx >= 16 && lx <= 512 && (ly & (ly - 1)) == 0 && (lx & (lx - 1)) == 0 &&
+         ly * lx >= 1024 && ly * lx <= (kind == KIND_F32 ? PLANE_F32_MAX : kind == KIND_SPLIT ? PLANE_SPLIT_MAX : PLANE_F64_MAX);
 }
 
+bool plane_shape_supported(long long ly, long long lx, int kind) { return plane_shape_ok(ly, lx, kind); }
+
 template <int LY, int LX, bool SPLIT, typename R>
-static void launch_shape(const PlaneArgs& a, hipStream_t s) {
-  if constexpr (sizeof(R) == 8) {
-    if constexpr (LY * LX <= PLANE_F64_MAX) {
-      const dim3 g((unsigned)a.nplanes), t(PlaneGeom<LY, LX, false>::NT);
-      if (a.inverse) FFTAMD_LAUNCH((k_fft_plane<LY, LX, true, false, double>), g, t, 0, s, a);
-      else FFTAMD_LAUNCH((k_fft_plane<LY, LX, false, false, double>), g, t, 0, s, a);
-    }
-    return;
+static bool launch_shape(const PlaneArgs& a, hipStream_t s) {
+  constexpr int kind = sizeof(R) == 8 ? KIND_F64 : SPLIT ? KIND_SPLIT : KIND_F32;
+  if constexpr (!plane_shape_ok(LY, LX, kind)) {
+    return false;
+  } else if constexpr (kind == KIND_F64) {
+    const dim3 g((unsigned)a.nplanes), t(PlaneGeom<LY, LX, false>::NT);
+    if (a.inverse) FFTAMD_LAUNCH((k_fft_plane<LY, LX, true, false, double>), g, t, 0, s, a);
+    else FFTAMD_LAUNCH((k_fft_plane<LY, LX, false, false, double>), g, t, 0, s, a);
+    return true;
   } else {
     launch_shape_f32<LY, LX, SPLIT>(a, s);
+    return true;
   }
 }
 
 template <int LY, bool SPLIT, typename R>
 static bool dispatch_lx(int lx, const PlaneArgs& a, hipStream_t s) {
   switch (lx) {
-    case 16: if constexpr (LY * 16 >= 1024) { launch_shape<LY, 16, SPLIT, R>(a, s); return true; } else return false;
-    case 32: if constexpr (LY * 32 >= 1024) { launch_shape<LY, 32, SPLIT, R>(a, s); return true; } else return false;
-    case 64: launch_shape<LY, 64, SPLIT, R>(a, s); return true;
-    case 128: launch_shape<LY, 128, SPLIT, R>(a, s); return true;
+    case 16: return launch_shape<LY, 16, SPLIT, R>(a, s);
+    case 32: return launch_shape<LY, 32, SPLIT, R>(a, s);
+    case 64: return launch_shape<LY, 64, SPLIT, R>(a, s);
+    case 128: return launch_shape<LY, 128, SPLIT, R>(a, s);
+    case 256: return launch_shape<LY, 256, SPLIT, R>(a, s);
+    case 512: return launch_shape<LY, 512, SPLIT, R>(a, s);
     default: return false;
   }
 }
@@ -192,6 +205,8 @@ static bool dispatch_ly(int ly, int lx, const PlaneArgs& a, hipStream_t s) {
     case 32: return dispatch_lx<32, SPLIT, R>(lx, a, s);
     case 64: return dispatch_lx<64, SPLIT, R>(lx, a, s);
     case 128: return dispatch_lx<128, SPLIT, R>(lx, a, s);
+    case 256: return dispatch_lx<256, SPLIT, R>(lx, a, s);
+    case 512: return dispatch_lx<512, SPLIT, R>(lx, a, s);
     default: return false;
   }
 }
@@ -200,7 +215,7 @@ void preload_plane() { preload_kernel(reinterpret_cast<const void*>(&k_fft_plane
 
 int launch_fft_plane(int ly, int lx, const PlaneArgs& a, void* stream, bool split, int prec) {
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  if (!plane_shape_supported(ly, lx, prec) || (prec == PREC_F64 && (split || a.w_load || a.w_store)) || a.nplanes == 0 || a.nplanes > 0xFFFFFFFFull / 1024 ||
+  if (!plane_shape_ok(ly, lx, pass_kind(split, prec)) || (prec == PREC_F64 && (split || a.w_load || a.w_store)) || a.nplanes == 0 || a.nplanes > 0xFFFFFFFFull / 1024 ||
       (a.tab && a.ppt == 0))
     return -1;
   const bool ok = prec == PREC_F64 ? dispatch_ly<false, double>(ly, lx, a, s)

@@ -12,7 +12,7 @@ namespace fftamd {
 
 template <int LY, int LX, bool SPLIT>
 struct PlaneGeom {
-  static_assert(LY >= 16 && LX >= 16 && LY <= 128 && LX <= 128, "plane sides 16..128");
+  static_assert(LY >= 16 && LX >= 16 && LY <= 512 && LX <= 512, "plane sides 16..512");
   using GX = Geom<LX, MODE_CONTIG, LY>;    // rows: LY lines of LX points
   using GY = Geom<LY, MODE_STRIDED, LX>;   // columns: LX lines of LY points
   static constexpr int NT = LY * LX / 16;
