@@ -382,7 +382,7 @@ static int split_natural(int prec, int lg, int* lg1, int* lg2) {
   const int m = ilog2c(lmax_strided_fourstep(prec));
   if (split_contig(prec, lg, lg1, lg2)) return -1;
   int a = std::min((lg + 1) / 2, m);
-  if (prec == PREC_F32 && (lg == 21 || lg == 22)) a = lg - 12;
+  if (prec == PREC_F32 && lg == 22) a = lg - 12;
   *lg1 = a;
   *lg2 = lg - a;
   return 0;
@@ -416,11 +416,11 @@ static constexpr unsigned long long plane_min_count(long long ly, long long lx) 
 }
 // most planes of one launch (grid size in work-items is 32-bit)
 static constexpr unsigned long long PLANE_MAX_COUNT = 0xFFFFFFFFull / 1024;
-// Fewest 16-column groups for which the one-pass 4096-point column transform
-// replaces the four-step pair (four workgroups per group, as the 256 x 256
-// plane pass): measured 29.5 against 31.2 us at 32 groups (4096 x 512), 39.9
-// against 32.9 us at 64 (4096 x 1024), 137.6 against 103.3 us at 4096 x 4096.
-static constexpr unsigned long long COL4096_MIN_GROUPS = 64;
+// Fewest 16-column groups for which the one-pass column transform replaces the
+// four-step pair: measured with the row pass, pair against one pass, 4096 rows
+// 30.3 and 32.4 us at 32 groups, 41.0 and 38.2 at 64, 78.6 and 66.9 at 128; 2048
+// rows 23.5 and 23.6 at 32, 32.3 and 28.7 at 64, 78.9 and 61.0 at 256.
+static constexpr unsigned long long COL_MIN_GROUPS = 64;
 
 // split mode applies to lines with a radix-16 stage (16..4096 points)
 static bool line_split(bool split, int lg) { return split && lg >= 4 && lg <= 12; }
@@ -429,18 +429,18 @@ static int pass_cols(const PassDesc& p, bool split, int prec) {
   return geom_cols_launch(1 << p.lg, p.mode, pass_kind(line_split(split, p.lg), prec), p.nouter * p.K * p.ncol);
 }
 
-// the 4096-point axis at element stride lx of `outer` arrays in one pass
-static PassDesc col4096_pass(long long lx, unsigned long long outer) {
+// an axis of l points (4096 or 2048) at element stride lx of `outer` arrays in one pass
+static PassDesc col_pass(int l, long long lx, unsigned long long outer) {
   PassDesc p;
-  p.lg = 12;
-  p.mode = MODE_COL4096;
+  p.lg = ilog2c(l);
+  p.mode = MODE_COL;
   p.transposing = true;  // the workgroups of a column group all read all of it
   p.in_p = p.out_p = lx;
   p.in_c = p.out_c = 1;
   p.ncol = (unsigned)lx;
   p.K = 1;
   p.nouter = outer;
-  p.in_o = p.out_o = 4096 * lx;
+  p.in_o = p.out_o = l * lx;
   return p;
 }
 
@@ -521,17 +521,18 @@ static int build_plan(int rank, const size_t* dims, size_t batch, unsigned flags
     }
   }
 
-  // a 4096-point second-fastest axis in one pass (four workgroups per group of
+  // a 4096- or 2048-point second-fastest axis in one pass (workgroups per group of
   // 16 columns, out of place), placed first so that the contiguous pass after
   // it runs in place on the output
   int col_axis = -1;
   if (rank >= 2 && top == rank - 1 && prec == PREC_F32 && !plan.split && !(flags & FLAG_NO_PLANE_FUSION) &&
-      dims[rank - 2] == 4096) {
+      (dims[rank - 2] == 4096 || dims[rank - 2] == 2048)) {
     const long long LX = (long long)dims[rank - 1];
     unsigned long long O = batch;
     for (int d = 0; d < rank - 2; ++d) O *= dims[d];
-    if (col4096_supported(LX, O) && (unsigned long long)(LX / 16) * O >= COL4096_MIN_GROUPS) {
-      ps.push_back(col4096_pass(LX, O));
+    const int LY = (int)dims[rank - 2];
+    if (col_supported(LY, LX, O) && (unsigned long long)(LX / 16) * O >= COL_MIN_GROUPS) {
+      ps.push_back(col_pass(LY, LX, O));
       col_axis = rank - 2;
     }
   }
@@ -539,7 +540,7 @@ static int build_plan(int rank, const size_t* dims, size_t batch, unsigned flags
   // an axis of L points at element stride st (st > 1) of O arrays: one strided
   // pass up to lmax points, the 4096-point column pass for the second half of
   // a long contiguous axis (out of place), else a four-step pair
-  auto push_strided = [&](long long L, long long st, unsigned long long O, int lmax) -> int {
+  auto push_strided = [&](long long L, long long st, unsigned long long O, int lmax, bool col) -> int {
     const int lg = ilog2c(L);
     if (L <= lmax) {
       PassDesc p;
@@ -557,9 +558,9 @@ static int build_plan(int rank, const size_t* dims, size_t batch, unsigned flags
       ps.push_back(p);
       return 0;
     }
-    if (lmax > lmax_strided(prec) && L == 4096 && prec == PREC_F32 && !plan.split &&
-        !(flags & FLAG_NO_PLANE_FUSION) && col4096_supported(st, O)) {
-      ps.push_back(col4096_pass(st, O));
+    if (col && prec == PREC_F32 && !plan.split && !(flags & FLAG_NO_PLANE_FUSION) && L <= 4096 &&
+        col_supported((int)L, st, O)) {
+      ps.push_back(col_pass((int)L, st, O));
       return 0;
     }
     int lg1, lg2;
@@ -650,7 +651,7 @@ static int build_plan(int rank, const size_t* dims, size_t batch, unsigned flags
           A.out_c = L1;
           A.transposing = true;
           ps.push_back(A);
-          if (push_strided(L2, L1, O, lmax_strided_fourstep(prec))) return -1;
+          if (push_strided(L2, L1, O, lmax_strided_fourstep(prec), true)) return -1;
           continue;
         }
         ps.push_back(A);  // in place
@@ -673,7 +674,11 @@ static int build_plan(int rank, const size_t* dims, size_t batch, unsigned flags
         ps.push_back(B);
       }
     } else {
-      if (push_strided(L, s, O, lmax_strided(prec))) return -1;
+      // 1024-point axes of 2D arrays (FP64: 512 and 1024 points of any) in one pass
+      // instead of a four-step pair: 1024 x 1024 21.1 -> 17.0 us, 16 x (1024 x 512)
+      // 78.9 -> 61.3, FP64 512 x 512 18.5 -> 12.7, 4 x (1024 x 1024) 80.4 -> 60.7
+      if (push_strided(L, s, O, rank == 2 || prec == PREC_F64 ? lmax_strided_fourstep(prec) : lmax_strided(prec), false))
+        return -1;
     }
   }
 
@@ -888,18 +893,18 @@ static int run_plan(Plan& plan, const void* din, void* dout, bool inverse, hipSt
       cur = p.dst;
       continue;
     }
-    if (p.mode == MODE_COL4096) {
+    if (p.mode == MODE_COL) {
       ColArgs ca{};
+      ca.l = 1 << p.lg;
       ca.in = ptr(p.src);
       ca.out = ptr(p.dst);
       ca.lx = p.in_p;
       ca.in_o = p.in_o;
       ca.ngroups = (unsigned)(p.ncol / 16);
       ca.nitems = p.nouter * ca.ngroups;
-      if (tab_stockham(plan, 256, &ca.tw)) return -1;
       if (tab_direct(plan, 256, &ca.w256)) return -1;
-      if (tab_fourstep(plan, 4096, &ca.ptw_lo, &ca.ptw_hi)) return -1;
-      ca.ptw_hb = fourstep_hb(4096);
+      if (tab_fourstep(plan, ca.l, &ca.ptw_lo, &ca.ptw_hi)) return -1;
+      ca.ptw_hb = fourstep_hb(ca.l);
       ca.w_load = pi == 0 ? w_load : nullptr;
       ca.w_store = pi + 1 == plan.passes.size() ? w_store : nullptr;
       ca.w_mask = (unsigned long long)plan.per - 1ULL;
@@ -907,14 +912,14 @@ static int run_plan(Plan& plan, const void* din, void* dout, bool inverse, hipSt
       Prof& pf = P();
       const bool prof = pf.on && !resolve && pf.used + 2 <= pf.pool.size();
       if (prof) HIP_TRY(hipEventRecord(pf.pool[pf.used], stream));
-      const int rc = launch_fft_col4096(ca, stream);
+      const int rc = launch_fft_col(ca, stream);
       if (prof) {
         HIP_TRY(hipEventRecord(pf.pool[pf.used + 1], stream));
-        pf.recs.push_back({"fft_col_f32_4096", pf.pool[pf.used], pf.pool[pf.used + 1]});
+        pf.recs.push_back({"fft_col_f32_" + std::to_string(ca.l), pf.pool[pf.used], pf.pool[pf.used + 1]});
         pf.used += 2;
       }
       if (rc) {
-        set_error("4096-point column pass launch failed (rc=%d): %s", rc, hipGetErrorString(hipGetLastError()));
+        set_error("%d-point column pass launch failed (rc=%d): %s", ca.l, rc, hipGetErrorString(hipGetLastError()));
         return -1;
       }
       cur = p.dst;
@@ -1993,12 +1998,12 @@ int describe_plan(int rank, const size_t* dims, size_t batch, unsigned flags, in
                        d.in_k, d.out_k, d.in_o, d.out_o, d.ncol, d.K, d.kbits,
                        (long long)d.nouter, d.M, d.cshift, d.src, d.dst,
                        d.mode == MODE_PLANE ? (d.K == 256 && d.lg == 8 ? 64 : (long long)d.K)
-                       : d.mode == MODE_COL4096 ? 16
+                       : d.mode == MODE_COL ? 16
                        : d.mode == MODE_CUBE_A ? (d.lg == 9 ? 64 : (1LL << d.lg) / 4)   // rows per workgroup
                        : d.mode == MODE_CUBE_B ? (d.lg == 9 ? 8 : d.lg == 8 || prec == PREC_F64 ? 16 : 32)   // columns per workgroup (x 8 or 4 rows x n planes)
                        : pass_cols(d, p.split, prec),
                        d.mode == MODE_PLANE ? plane_threads(d)
-                       : d.mode == MODE_COL4096 ? 512
+                       : d.mode == MODE_COL ? 1024
                        : d.mode == MODE_CUBE_A ? (d.lg == 9 ? 1024 : d.lg == 8 ? 512 : 256)
                        : d.mode == MODE_CUBE_B ? (d.lg == 9 ? 1024 : prec == PREC_F64 ? 256 : 512)
                        : pass_cols(d, p.split, prec) * geom_tpl(1 << d.lg)};

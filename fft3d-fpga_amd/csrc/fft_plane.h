@@ -36,19 +36,19 @@ constexpr long long PLANE_F32_MAX = 32768, PLANE_SPLIT_MAX = 16384, PLANE_F64_MA
 int launch_fft_plane(int ly, int lx, const PlaneArgs& a, void* stream, bool split = false, int prec = 0);
 bool plane_shape_supported(long long ly, long long lx, int kind);  // kind: PassKind
 
-// The 4096-point transform along the second-fastest axis of blocks of 4096
-// rows of lx elements (fft_col.hip): element (o, row, x) at o * in_o + row *
-// lx + x.  Four workgroups per group of 16 adjacent columns.
+// The l-point transform (l = 4096 or 2048) along the second-fastest axis of
+// blocks of l rows of lx elements (fft_col.hip): element (o, row, x) at o * in_o
+// + row * lx + x.  l / 2048 workgroups per group of 16 adjacent columns.
 struct ColArgs {
   const void* in;
   void* out;
+  int l;
   long long lx;                  // row length in complex elements (multiple of 16)
-  long long in_o;                // elements between blocks (4096 * lx)
+  long long in_o;                // elements between blocks (l * lx)
   unsigned long long nitems;     // blocks x column groups
   unsigned ngroups;              // column groups per block (lx / 16)
-  const void* tw;                // Stockham twiddles of 256-point lines
   const void* w256;              // W256^m, m = 0..255
-  const void* ptw_lo;            // W4096^t = ptw_hi[t >> ptw_hb] * ptw_lo[t & (2^ptw_hb - 1)]
+  const void* ptw_lo;            // W_l^t = ptw_hi[t >> ptw_hb] * ptw_lo[t & (2^ptw_hb - 1)]
   const void* ptw_hi;
   unsigned ptw_hb;
   const float* w_load;           // optional real weights (see PassArgs)
@@ -59,8 +59,8 @@ struct ColArgs {
 
 // 0 on success, -1 for an unsupported shape or grid, -2 on a launch error.
 // Out of place only: in and out must not overlap.
-int launch_fft_col4096(const ColArgs& a, void* stream);
-bool col4096_supported(long long lx, unsigned long long nouter);
+int launch_fft_col(const ColArgs& a, void* stream);
+bool col_supported(int l, long long lx, unsigned long long nouter);
 
 // Arrays of n x n x n blocks (n = 512, 256 or 128) in two passes with the y
 // axis split between them: (n/4) x 4 for n = 256 and 128 (fft_cube.hip),

@@ -51,7 +51,7 @@ extern "C" {
 /* Single-precision transforms whose two fastest axes form planes up to
  * 128 x 128, or 256 x 256 (from 32 planes up), run both axes in one fused pass
  * over each plane (a 3D transform then reads and writes HBM twice, not three
- * times); a second-fastest axis of 4096 points (from 64 groups of 16 columns
+ * times); a second-fastest axis of 2048 or 4096 points (from 64 groups of 16 columns
  * up) runs in one pass instead of a four-step pair.  This flag asks for the
  * separate line passes instead (it also turns off the y-split pair below). */
 #define FFTAMD_NO_PLANE_FUSION 0x4u

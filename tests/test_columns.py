@@ -1,0 +1,112 @@
+"""Long second-fastest axes: the one-pass 2048- and 4096-point column kernel
+(two workgroups per group of columns at 4096), and 1024-point (FP64 512- and
+1024-point) axes in one strided pass.  The column kernel's row, LDS and output
+maps are replayed on the CPU, plans against the oracle, the kernels on the GPU
+at the fewest groups that take them, odd batches, weights, unaligned input."""
+import numpy as np
+import pytest
+from test_plan_sim import describe, run_plan, sched
+
+
+def emulate_columns(x):
+    """k_fft_col's maps for the 16 columns of one group (x: L x 16)."""
+    L = x.shape[0]
+    Q, N1 = L // 2048, L // 16
+    PER, LH, TPL = N1 // 64, 8 // Q, N1 // 16
+    _, rad, ns = sched(N1)
+    assert ns[1] == TPL and L // TPL == 256
+    w = lambda M, t: np.exp(-2j * np.pi * (t % M) / M)  # noqa: E731
+    out = np.full_like(x, np.nan)
+    for grp in (0, 1, 3):
+        reads = []
+        for P in range(Q):
+            lines = np.full((16, N1, 16), np.nan + 0j)  # [u][n1][column]: the first-stage outputs
+            for gi in range(64):
+                for i in range(PER):
+                    n1 = gi + 64 * (((i ^ P) + (grp & (PER - 1))) & (PER - 1))
+                    reads.append((P, n1))
+                    y = np.fft.fft(x[n1 + N1 * np.arange(16)], axis=0)  # k1 = P + Q u
+                    assert np.isnan(lines[: 16 // Q, n1]).all()
+                    lines[: 16 // Q, n1] = y[P::Q]
+            for h in range(2):
+                for lane in range(LH):
+                    k1 = P + Q * (LH * h + lane)
+                    z = lines[LH * h + lane]
+                    for tau in range(TPL):  # W_L^{n1 k1} as W_L^{tau k1} W256^{m k1}
+                        for b in range(16 // rad[0]):
+                            for r in range(rad[0]):
+                                n1, m = tau + b * TPL + r * (N1 // rad[0]), b + r * (N1 // rad[0] // TPL)
+                                assert n1 == tau + TPL * m and tau * k1 < 256
+                                assert np.isclose(w(L, n1 * k1), w(L, tau * k1) * w(256, m * k1))
+                    z = np.fft.fft(z * w(L, np.arange(N1) * k1)[:, None], axis=0)
+                    for tau in range(TPL):
+                        for r in range(16):
+                            row = (k1 + 16 * tau) + 16 * TPL * r
+                            if grp == 0:
+                                assert np.isnan(out[row]).all()
+                            out[row] = z[tau + TPL * r]
+        assert len(set(reads)) == len(reads) == Q * N1
+    return out
+
+
+@pytest.mark.parametrize("L", [2048, 4096])
+def test_column_maps(L):
+    r = np.random.default_rng(L)
+    x = r.standard_normal((L, 16)) + 1j * r.standard_normal((L, 16))
+    assert np.allclose(emulate_columns(x), np.fft.fft(x, axis=0), atol=1e-9)
+
+
+@pytest.mark.parametrize("dims,batch,flags,prec,modes", [
+    ([2048, 1024], 1, 0, 0, [3, 0]), ([2048, 512], 2, 0, 0, [3, 0]), ([2048, 512], 1, 0, 0, [0, 1, 1]),
+    ([2048, 1024], 1, 2, 0, [0, 1, 1]), ([2048, 1024], 1, 4, 0, [0, 1, 1]), ([2, 2048, 512], 1, 0, 0, [3, 0, 1]),
+    ([1024, 64], 3, 0, 0, [0, 1]), ([1024, 64], 1, 2, 0, [0, 1]), ([1024, 32], 1, 0, 1, [0, 1]), ([512, 32], 2, 0, 1, [0, 1]),
+    ([2, 512, 32], 1, 0, 1, [0, 1, 1]), ([2048, 16], 1, 0, 1, [0, 1, 1])])
+@pytest.mark.parametrize("inverse", [False, True])
+@pytest.mark.parametrize("aliased", [False, True])
+def test_plans(fl, orc, dims, batch, flags, prec, modes, inverse, aliased):
+    passes, final_copy = describe(fl, dims, batch, flags, prec=prec, aliased=aliased)
+    assert [p["mode"] for p in passes] == modes
+    x = orc.uniform(int(np.prod(dims)) * batch, 61)
+    got = run_plan(passes, final_copy, x, inverse, aliased=aliased)
+    ref = orc.fftnd(x, dims, batch=batch, inverse=inverse).reshape(-1)
+    assert np.linalg.norm(got - ref) <= 1e-12 * np.linalg.norm(ref)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape,dtype,split", [
+    ((2048, 1024), "complex64", False), ((3, 2048, 512), "complex64", False), ((65, 2048, 16), "complex64", False),
+    ((4096, 1024), "complex64", False), ((67, 4096, 16), "complex64", False), ((3, 1024, 64), "complex64", False),
+    ((1024, 1024), "complex64", False), ((2, 1024, 32), "complex64", True), ((3, 512, 64), "complex128", False),
+    ((1024, 32), "complex128", False), ((5, 1024, 8), "complex128", False)])
+def test_vs_oracle(gpu_lib, orc, shape, dtype, split):
+    import torch
+    dims, n = list(shape[-2:]), int(np.prod(shape))
+    batch = n // int(np.prod(dims))
+    x = orc.gauss(n, 71).astype(dtype)
+    tol = 1e-14 if dtype == "complex128" else 2e-6
+    for inv in (False, True):
+        ref = orc.fftnd(x, dims, batch=batch, inverse=inv).reshape(batch, -1)
+        # one element into an allocation: an input off the 16-byte boundary
+        base = torch.zeros(n + 1, dtype=getattr(torch, dtype), device="cuda")
+        base[1:] = torch.from_numpy(x).cuda()
+        xt = base[1:].view(batch, *dims)
+        y = gpu_lib.c2c_dev(xt, 2, inverse=inv, split=split)
+        gpu_lib.c2c_dev(xt, 2, inverse=inv, split=split, out=xt)
+        assert torch.equal(xt, y)
+        d = np.linalg.norm(y.cpu().numpy().reshape(batch, -1) - ref, axis=1) / np.linalg.norm(ref, axis=1)
+        print(f"{shape} {dtype} split={split} inv={inv} worst {d.max():.3e}", flush=True)
+        assert d.max() <= tol
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("ly,lx,batch", [(2048, 512, 2), (4096, 1024, 1), (1024, 32, 3)])
+def test_weights(gpu_lib, orc, ly, lx, batch):
+    import torch
+    from fftfpga_amd.autograd import weighted_transform
+    x = orc.gauss(batch * ly * lx, 3).reshape(batch, ly, lx)
+    w = np.abs(orc.uniform(ly * lx, 4).real).reshape(ly, lx).astype(np.float32)
+    xt, wt = torch.from_numpy(x).cuda(), torch.from_numpy(w).cuda()
+    out = weighted_transform(xt, 2, w_in=wt, w_out=wt).cpu().numpy()
+    assert orc.rel_l2(out, orc.fftnd((x * w).reshape(-1), [ly, lx], batch=batch) * w) <= 2e-6
+    out = weighted_transform(xt, 2, inverse=True, w_out=wt).cpu().numpy()
+    assert orc.rel_l2(out, orc.fftnd(x.reshape(-1), [ly, lx], batch=batch, inverse=True) * w) <= 2e-6
