@@ -138,6 +138,23 @@ def load(path: str | None = None) -> ctypes.CDLL:
     return lib
 
 
+_raw_stream = None
+
+
+def stream_handle(device) -> int:
+    """hipStream_t of torch's current stream on `device`, as an int.
+
+    torch.cuda.current_stream builds a Stream object (2.0 us a call); the raw
+    handle alone takes 0.15 us, where this torch has that call.
+    """
+    global _raw_stream
+    if _raw_stream is None:
+        import torch
+        _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream",
+                              lambda index: torch.cuda.current_stream(index).cuda_stream)
+    return _raw_stream(device.index)
+
+
 def last_error() -> str:
     msg = load().fftamd_last_error()
     return msg.decode() if msg else ""

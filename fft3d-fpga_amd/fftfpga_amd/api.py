@@ -13,10 +13,11 @@ on the current torch stream.
 from __future__ import annotations
 
 import ctypes
+import math
 
 import numpy as np
 
-from ._lib import FpgaT, last_error, load
+from ._lib import FpgaT, last_error, load, stream_handle
 
 FFTAMD_BITREV_1D = 0x1
 FFTAMD_SPLIT_MFMA = 0x2
@@ -135,11 +136,6 @@ def fftfpgaf_c2c_3d_ddr_svm_batch(N, inp, out, inv=False, how_many=2) -> FpgaT:
 
 # ---- device-pointer transforms (torch tensors on the GPU) -------------------------
 
-def _stream_handle(t) -> ctypes.c_void_p:
-    import torch
-    return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
-
-
 def c2c_dev(x, rank: int, inverse: bool = False, bitrev_1d: bool = False, out=None,
             split: bool = False, plane_fusion: bool = True, cube_split: bool = True):
     """Transform the last `rank` dims of a contiguous complex64/complex128 GPU
@@ -159,10 +155,9 @@ def c2c_dev(x, rank: int, inverse: bool = False, bitrev_1d: bool = False, out=No
         raise ValueError("contiguous tensor expected")
     if rank < 1 or rank > 3 or x.dim() < rank:
         raise ValueError("bad rank")
-    dims = [int(d) for d in x.shape[x.dim() - rank:]]
-    batch = 1
-    for d in x.shape[: x.dim() - rank]:
-        batch *= int(d)
+    shape = x.shape
+    dims = shape[len(shape) - rank:]
+    batch = math.prod(shape[:len(shape) - rank])
     if out is None:
         out = torch.empty_like(x)
     elif out.shape != x.shape or out.dtype != x.dtype or not out.is_contiguous():
@@ -173,8 +168,7 @@ def c2c_dev(x, rank: int, inverse: bool = False, bitrev_1d: bool = False, out=No
     fn = load().fftamd_c2c_dev if x.dtype == torch.complex64 else load().fftamd_z2z_dev
     flags = ((FFTAMD_BITREV_1D if bitrev_1d else 0) | (FFTAMD_SPLIT_MFMA if split else 0)
              | (0 if plane_fusion else FFTAMD_NO_PLANE_FUSION) | (0 if cube_split else FFTAMD_NO_CUBE_SPLIT))
-    rc = fn(rank, cd, batch, ctypes.c_void_p(x.data_ptr()), ctypes.c_void_p(out.data_ptr()),
-            1 if inverse else 0, flags, _stream_handle(x))
+    rc = fn(rank, cd, batch, x.data_ptr(), out.data_ptr(), 1 if inverse else 0, flags, stream_handle(x.device))
     if rc != 0:
         raise RuntimeError(f"fftamd transform failed: {last_error()}")
     return out

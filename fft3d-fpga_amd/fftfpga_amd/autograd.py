@@ -19,11 +19,7 @@ import math
 
 import torch
 
-from ._lib import last_error, load
-
-
-def _stream(t):
-    return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+from ._lib import last_error, load, stream_handle
 
 
 def _check(x, rank):
@@ -37,23 +33,21 @@ def weighted_transform(x, rank, inverse=False, w_in=None, w_out=None, out=None):
     """out = w_out . F(w_in . x) on the current stream (no autograd)."""
     _check(x, rank)
     x = x.contiguous()
-    dims = [int(d) for d in x.shape[x.dim() - rank:]]
-    batch = x.numel() // max(1, int(torch.tensor(dims).prod().item()))
+    dims = x.shape[x.dim() - rank:]
+    batch = x.numel() // max(1, math.prod(dims))
     if out is None:
         out = torch.empty_like(x)
     for w in (w_in, w_out):
-        if w is not None and (w.dtype != torch.float32 or not w.is_cuda or list(w.shape) != dims
+        if w is not None and (w.dtype != torch.float32 or not w.is_cuda or w.shape != dims
                               or not w.is_contiguous()):
             raise ValueError("weights must be contiguous float32 CUDA/HIP tensors of the transform shape")
     if batch == 0:
         return out
     cd = (ctypes.c_uint * rank)(*dims)
     rc = load().fftamd_c2c_weighted_dev(
-        rank, cd, batch, ctypes.c_void_p(x.data_ptr()), ctypes.c_void_p(out.data_ptr()),
-        1 if inverse else 0,
-        ctypes.c_void_p(w_in.data_ptr()) if w_in is not None else None,
-        ctypes.c_void_p(w_out.data_ptr()) if w_out is not None else None,
-        _stream(x))
+        rank, cd, batch, x.data_ptr(), out.data_ptr(), 1 if inverse else 0,
+        w_in.data_ptr() if w_in is not None else None, w_out.data_ptr() if w_out is not None else None,
+        stream_handle(x.device))
     if rc != 0:
         raise RuntimeError(f"fftamd weighted transform failed: {last_error()}")
     return out
@@ -62,7 +56,7 @@ def weighted_transform(x, rank, inverse=False, w_in=None, w_out=None, out=None):
 def weight_gradient(g, fx, rank):
     """Re sum over the batch of conj(g) . fx, one float per point of a transform (no autograd)."""
     _check(fx, rank)
-    dims = [int(d) for d in fx.shape[fx.dim() - rank:]]
+    dims = fx.shape[fx.dim() - rank:]
     # a lazily conjugated or negated gradient is made plain: the kernel reads its memory
     g, fx = g.resolve_conj().resolve_neg().contiguous(), fx.contiguous()
     if g.dtype != fx.dtype or g.shape != fx.shape or g.device != fx.device:
@@ -72,8 +66,8 @@ def weight_gradient(g, fx, rank):
         return torch.zeros(dims, dtype=torch.float32, device=fx.device)
     gw = torch.empty(dims, dtype=torch.float32, device=fx.device)
     cd = (ctypes.c_uint * rank)(*dims)
-    rc = load().fftamd_weight_grad_dev(rank, cd, fx.numel() // points, ctypes.c_void_p(g.data_ptr()),
-                                       ctypes.c_void_p(fx.data_ptr()), ctypes.c_void_p(gw.data_ptr()), _stream(fx))
+    rc = load().fftamd_weight_grad_dev(rank, cd, fx.numel() // points, g.data_ptr(), fx.data_ptr(), gw.data_ptr(),
+                                       stream_handle(fx.device))
     if rc != 0:
         raise RuntimeError(f"fftamd weight gradient failed: {last_error()}")
     return gw

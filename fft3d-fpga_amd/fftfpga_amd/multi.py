@@ -28,13 +28,9 @@ import os
 
 import torch
 
-from ._lib import XForm3D, last_error, load
+from ._lib import XForm3D, last_error, load, stream_handle
 
 DEFAULT_TUNE_CACHE = os.path.join(os.path.expanduser("~"), ".cache", "fftamd", "tune.txt")
-
-
-def _stream(dev=None):
-    return ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
 
 
 def packed_offsets(shapes):
@@ -78,18 +74,18 @@ class MultiPlan:
         self.device = d_in.device
 
     def __call__(self):
-        if self._lib.fftamd_multi_exec(self._h, _stream(self.device)) != 0:
+        if self._lib.fftamd_multi_exec(self._h, stream_handle(self.device)) != 0:
             raise RuntimeError(f"fftamd_multi_exec failed: {last_error()}")
 
     def check(self):
-        if self._lib.fftamd_multi_check(self._h, _stream(self.device)) != 0:
+        if self._lib.fftamd_multi_check(self._h, stream_handle(self.device)) != 0:
             raise RuntimeError(f"multi-transform launch reported: {last_error()}")
 
     def tune(self, cache_path: str | None = DEFAULT_TUNE_CACHE, reps: int = 3):
         if cache_path:
             os.makedirs(os.path.dirname(cache_path), exist_ok=True)
         us = ctypes.c_double(0)
-        rc = self._lib.fftamd_multi_tune(self._h, _stream(self.device),
+        rc = self._lib.fftamd_multi_tune(self._h, stream_handle(self.device),
                                          cache_path.encode() if cache_path else None, reps,
                                          ctypes.byref(us))
         if rc < 0:
