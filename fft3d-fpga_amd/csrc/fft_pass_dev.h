@@ -40,7 +40,9 @@ struct Geom {
 };
 
 // TAB: split stages read their constant operands from the LDS table `atab`
-template <typename R, int L, int MODE, int S, bool SPLIT = false, int CC = geom_cols(L, MODE), bool TAB = false>
+// PRE: tw already points at this thread's four table powers
+template <typename R, int L, int MODE, int S, bool SPLIT = false, int CC = geom_cols(L, MODE), bool TAB = false,
+          bool PRE = false>
 __device__ __forceinline__ void stage_compute(cpx<R>* v, int tau, const cpx<R>* __restrict__ tw,
                                               cpx<R>* lds = nullptr, const split_half8* atab = nullptr) {
   using G = Geom<L, MODE, CC>;
@@ -55,7 +57,7 @@ __device__ __forceinline__ void stage_compute(cpx<R>* v, int tau, const cpx<R>* 
       const int j = tau + b * G::TPL;
       const int k = j & (NS - 1);
       // W^k, W^2k, W^4k, W^8k from the table; W^{kr} for the other r by products
-      const cpx<R>* t = tw + OFF + TW_PER_K * k;
+      const cpx<R>* t = PRE ? tw : tw + OFF + TW_PER_K * k;
       const cpx<R> w1 = t[0], w2 = t[1], w4 = t[2], w8 = t[3];
       const cpx<R> w3 = cmul(w1, w2), w12 = cmul(w4, w8);
       cpx<R> w[16];
@@ -118,20 +120,37 @@ __device__ __forceinline__ void stage_load_lds(cpx<R>* v, const cpx<R>* lds, int
   }
 }
 
-template <typename R, int L, int MODE, int S, bool SPLIT = false, int CC = geom_cols(L, MODE)>
+// this thread's four table powers of stage S (one radix-16 butterfly per thread)
+template <typename R, int L, int S>
+__device__ __forceinline__ void stage_twiddles(cpx<R>* t4, int tau, const cpx<R>* __restrict__ tw) {
+  if constexpr (S > 0 && S < sched_np(L)) {
+    const cpx<R>* t = tw + sched_twoff(L, S) + TW_PER_K * (tau & (sched_ns(L, S) - 1));
+#pragma unroll
+    for (int q = 0; q < TW_PER_K; ++q) t4[q] = t[q];
+  }
+}
+
+// AHEAD: the next stage's table powers are loaded before this stage's
+// arithmetic, so that they arrive behind it and the barrier and not after
+// (30000 x 256 points 28.5 -> 25.9 us, 10007 x 1024 37.3 -> 35.2, 2500 x 4096 38.4
+// -> 35.8, 160 x 64^3 251 -> 247); the kernels at their register limit load them
+// where they are used.
+template <typename R, int L, int MODE, int S, bool SPLIT = false, int CC = geom_cols(L, MODE), bool AHEAD = !SPLIT>
 __device__ __forceinline__ void run_stages(cpx<R>* v, cpx<R>* lds, int c, int tau,
-                                           const cpx<R>* __restrict__ tw) {
+                                           const cpx<R>* __restrict__ tw, const cpx<R>* pre = nullptr) {
   using G = Geom<L, MODE, CC>;
   if constexpr (S < G::NP) {
+    cpx<R> next[TW_PER_K];
+    if constexpr (AHEAD) stage_twiddles<R, L, S + 1>(next, tau, tw);
     if constexpr (S > 0) {
       __syncthreads();  // previous stage's LDS writes are visible
       stage_load_lds<R, L, MODE, S, CC>(v, lds, c, tau);
     }
-    stage_compute<R, L, MODE, S, SPLIT, CC>(v, tau, tw, lds);
+    stage_compute<R, L, MODE, S, SPLIT, CC, false, AHEAD && (S > 0)>(v, tau, AHEAD && S > 0 ? pre : tw, lds);
     if constexpr (S + 1 < G::NP) {
       if constexpr (S > 0) __syncthreads();  // every thread finished reading this stage
       stage_store_lds<R, L, MODE, S, CC>(v, lds, c, tau);
-      run_stages<R, L, MODE, S + 1, SPLIT, CC>(v, lds, c, tau, tw);
+      run_stages<R, L, MODE, S + 1, SPLIT, CC, AHEAD>(v, lds, c, tau, tw, next);
     }
   }
 }

@@ -99,7 +99,7 @@ __global__ void __launch_bounds__(LY * LX / 32, 4) k_fft_plane_halves(const Plan
       }
     }
     if (h) __syncthreads();  // the first half's last stage has read the buffer
-    run_stages<float, LX, MODE_CONTIG, 0, false, HY>(v, lds, rc, rtau, reinterpret_cast<const cpx<float>*>(a.tw_x));
+    run_stages<float, LX, MODE_CONTIG, 0, false, HY, false>(v, lds, rc, rtau, reinterpret_cast<const cpx<float>*>(a.tw_x));
   }
 
   // ---- columns, in two halves: thread (column c, tau), adjacent threads on adjacent columns
@@ -116,7 +116,7 @@ __global__ void __launch_bounds__(LY * LX / 32, 4) k_fft_plane_halves(const Plan
     cpx<float> v[16];
     stage_load_lds<float, LY, MODE_STRIDED, 0, HX>(v, lds, cc, ctau);
     __syncthreads();  // every thread holds its stage-0 inputs before stage 0 stores
-    run_stages<float, LY, MODE_STRIDED, 0, false, HX>(v, lds, cc, ctau, reinterpret_cast<const cpx<float>*>(a.tw_y));
+    run_stages<float, LY, MODE_STRIDED, 0, false, HX, false>(v, lds, cc, ctau, reinterpret_cast<const cpx<float>*>(a.tw_y));
     constexpr int NPY = GY::NP;
     constexpr int RL = sched_radix(LY, NPY - 1), NSL = sched_ns(LY, NPY - 1), NBL = 16 / RL;
 #pragma unroll
