@@ -414,6 +414,14 @@ static constexpr unsigned long long plane_min_count(long long ly, long long lx) 
   if (ly <= 128 && lx <= 128) return PLANE_MIN_COUNT;
   return ly * lx <= 4096 ? 1 : ly * lx <= 8192 ? 16 : ly * lx <= 16384 ? 128 : 256;
 }
+// Fewest boxes for which the one-pass box kernel (one workgroup per box)
+// replaces the passes per plane and axis: one up to 8192 points or where a plane
+// has no plane pass (one 16^3 box 3.5 against 11.4 us, one 64 x 16 x 16 8.7 against
+// 12.4); else 64 at 16384 points (one 16 x 32 x 32 box 10.1 against 6.5 us, 32 of
+// them 11.1 against 9.5, 128 13.8 against 18.6).
+static constexpr size_t box_min_count(size_t points, size_t plane) {
+  return points <= 8192 || plane < 1024 ? 1 : 64;
+}
 // most planes of one launch (grid size in work-items is 32-bit)
 static constexpr unsigned long long PLANE_MAX_COUNT = 0xFFFFFFFFull / 1024;
 // Fewest 16-column groups for which the one-pass column transform replaces the
@@ -493,6 +501,23 @@ static int build_plan(int rank, const size_t* dims, size_t batch, unsigned flags
     B.in_o = B.out_o = CN * CN * CN;
     ps.push_back(B);
     top = rank - 4;
+  }
+
+  // small boxes: all three axes in one pass
+  if (rank == 3 && top == rank - 1 && !plan.split && !(flags & FLAG_NO_PLANE_FUSION) &&
+      box_supported((long long)dims[0], (long long)dims[1], (long long)dims[2], prec) && batch <= BOX_MAX_COUNT &&
+      batch >= box_min_count(tot, dims[1] * dims[2])) {
+    PassDesc p;
+    p.lg = ilog2c((long long)dims[2]);
+    p.mode = MODE_BOX;
+    p.in_p = p.out_p = 1;
+    p.in_c = p.out_c = (long long)dims[2];
+    p.ncol = (unsigned)dims[0];
+    p.K = (unsigned)dims[1];
+    p.nouter = batch;
+    p.in_o = p.out_o = (long long)tot;
+    ps.push_back(p);
+    top = -1;
   }
 
   // planes of the two fastest axes in one fused x+y pass: 256 x 256 (four
@@ -855,6 +880,37 @@ static int run_plan(Plan& plan, const void* din, void* dout, bool inverse, hipSt
       cur = p.dst;
       continue;
     }
+    if (p.mode == MODE_BOX) {
+      const int LX = 1 << p.lg, LY = (int)p.K, LZ = (int)p.ncol;
+      BoxArgs ba{};
+      ba.in = ptr(p.src);
+      ba.out = ptr(p.dst);
+      ba.nboxes = p.nouter;
+      if (sched_np(LZ) > 1 && tab_stockham(plan, LZ, &ba.tw_z)) return -1;
+      if (sched_np(LY) > 1 && tab_stockham(plan, LY, &ba.tw_y)) return -1;
+      if (sched_np(LX) > 1 && tab_stockham(plan, LX, &ba.tw_x)) return -1;
+      ba.w_load = w_load;
+      ba.w_store = w_store;
+      ba.w_mask = (unsigned long long)plan.per - 1ULL;
+      ba.inverse = inverse ? 1 : 0;
+      Prof& pf = P();
+      const bool prof = pf.on && !resolve && pf.used + 2 <= pf.pool.size();
+      if (prof) HIP_TRY(hipEventRecord(pf.pool[pf.used], stream));
+      const int rc = launch_fft_box(LZ, LY, LX, ba, stream, plan.prec);
+      if (prof) {
+        HIP_TRY(hipEventRecord(pf.pool[pf.used + 1], stream));
+        char lab[64];
+        snprintf(lab, sizeof(lab), "fft_box_%s_%dx%dx%d", plan.prec == PREC_F64 ? "f64" : "f32", LZ, LY, LX);
+        pf.recs.push_back({lab, pf.pool[pf.used], pf.pool[pf.used + 1]});
+        pf.used += 2;
+      }
+      if (rc) {
+        set_error("box pass launch failed (rc=%d): %s", rc, hipGetErrorString(hipGetLastError()));
+        return -1;
+      }
+      cur = p.dst;
+      continue;
+    }
     if (p.mode == MODE_CUBE_A || p.mode == MODE_CUBE_B) {
       const bool A = p.mode == MODE_CUBE_A;
       CubeArgs ca{};
@@ -960,13 +1016,21 @@ static int run_plan(Plan& plan, const void* din, void* dout, bool inverse, hipSt
     const unsigned long long per_outer = (unsigned long long)a.ncb * a.K;
     const unsigned long long max_blocks = (0xFFFFFFFFULL / (unsigned)(C * geom_tpl(L)));
     const unsigned long long outer_per_launch = std::max(1ULL, max_blocks / per_outer);
-    for (unsigned long long o0 = 0; o0 < p.nouter; o0 += outer_per_launch) {
+    // columns of several outer indices share a tile where one has too few
+    const unsigned long long packed = (p.nouter * p.ncol + C - 1) / C;
+    const bool pack = p.mode == MODE_STRIDED && p.K == 1 && p.ncol < (unsigned)C && p.out_p != 1 && packed <= max_blocks;
+    if (pack) {
+      a.pack = 1 + (unsigned)ilog2c(p.ncol);
+      a.nlines = p.nouter * p.ncol;
+    }
+    for (unsigned long long o0 = 0; o0 < p.nouter; o0 += pack ? p.nouter : outer_per_launch) {
       const unsigned long long no = std::min(outer_per_launch, p.nouter - o0);
+      const unsigned long long blocks = pack ? packed : per_outer * no;
       a.outer0 = o0;
       Prof& pf = P();
       const bool prof = pf.on && !resolve && pf.used + 2 <= pf.pool.size();
       if (prof) HIP_TRY(hipEventRecord(pf.pool[pf.used], stream));
-      int rc = launch_fft_pass(plan.prec, p.lg, p.mode, p.epi, a, per_outer * no, stream, split);
+      int rc = launch_fft_pass(plan.prec, p.lg, p.mode, p.epi, a, blocks, stream, split);
       if (prof) {
         HIP_TRY(hipEventRecord(pf.pool[pf.used + 1], stream));
         char lab[96];
@@ -1876,6 +1940,7 @@ int runtime_init(int dev, bool svm) {
   preload_multi();
   preload_flow();
   preload_wgrad();
+  preload_box();
   st.dev = dev;
   st.svm = svm;
   st.ready = true;
@@ -1997,12 +2062,14 @@ int describe_plan(int rank, const size_t* dims, size_t batch, unsigned flags, in
     long long v[NF] = {d.lg, d.mode, d.epi, d.transposing, d.in_p, d.out_p, d.in_c, d.out_c,
                        d.in_k, d.out_k, d.in_o, d.out_o, d.ncol, d.K, d.kbits,
                        (long long)d.nouter, d.M, d.cshift, d.src, d.dst,
-                       d.mode == MODE_PLANE ? (d.K == 256 && d.lg == 8 ? 64 : (long long)d.K)
+                       d.mode == MODE_BOX ? 1
+                       : d.mode == MODE_PLANE ? (d.K == 256 && d.lg == 8 ? 64 : (long long)d.K)
                        : d.mode == MODE_COL ? 16
                        : d.mode == MODE_CUBE_A ? (d.lg == 9 ? 64 : (1LL << d.lg) / 4)   // rows per workgroup
                        : d.mode == MODE_CUBE_B ? (d.lg == 9 ? 8 : d.lg == 8 || prec == PREC_F64 ? 16 : 32)   // columns per workgroup (x 8 or 4 rows x n planes)
                        : pass_cols(d, p.split, prec),
-                       d.mode == MODE_PLANE ? plane_threads(d)
+                       d.mode == MODE_BOX ? (long long)d.ncol * (long long)(d.K << d.lg) / 16
+                       : d.mode == MODE_PLANE ? plane_threads(d)
                        : d.mode == MODE_COL ? 1024
                        : d.mode == MODE_CUBE_A ? (d.lg == 9 ? 1024 : d.lg == 8 ? 512 : 256)
                        : d.mode == MODE_CUBE_B ? (d.lg == 9 ? 1024 : prec == PREC_F64 ? 256 : 512)

@@ -16,6 +16,11 @@ struct PassArgs {
   unsigned K;             // middle extent
   unsigned kbits;         // nonzero: output middle offset uses bitrev(k, kbits)
   unsigned long long outer0;  // first outer index of this launch
+  // strided pass with fewer columns than a tile holds lines (K == 1, ncol a power
+  // of two): tiles run over the columns of consecutive outer indices, nlines in
+  // all; pack = 1 + log2(ncol), 0 otherwise
+  unsigned pack;
+  unsigned long long nlines;
   const void* tw;         // Stockham stage twiddles for this line length
   // four-step post-twiddle W_M^t: t = ((col >> cshift) * k) & (M-1) = hi*2^hb + lo
   const void* ptw_lo;

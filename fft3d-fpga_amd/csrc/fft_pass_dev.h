@@ -170,6 +170,15 @@ __device__ __forceinline__ TileLoc tile_locate(const PassArgs& a, unsigned long 
   TileLoc t;
   t.c = MODE == MODE_CONTIG ? tid / G::TPL : tid % G::C;
   t.tau = MODE == MODE_CONTIG ? tid % G::TPL : tid / G::C;
+  if (MODE == MODE_STRIDED && a.pack) {
+    const unsigned long long line = g * G::C + (unsigned)t.c;
+    const unsigned long long o = line >> (a.pack - 1);
+    t.col = (unsigned)line & (a.ncol - 1);
+    t.active = line < a.nlines;
+    t.in_off = (long long)o * a.in_o + (long long)t.col * a.in_c;
+    t.out_off = (long long)o * a.out_o + (long long)t.col * a.out_c;
+    return t;
+  }
   const unsigned cb = (unsigned)(g % a.ncb);
   g /= a.ncb;
   const unsigned kk = (unsigned)(g % a.K);

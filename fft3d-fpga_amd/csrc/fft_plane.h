@@ -36,6 +36,27 @@ constexpr long long PLANE_F32_MAX = 32768, PLANE_SPLIT_MAX = 16384, PLANE_F64_MA
 int launch_fft_plane(int ly, int lx, const PlaneArgs& a, void* stream, bool split = false, int prec = 0);
 bool plane_shape_supported(long long ly, long long lx, int kind);  // kind: PassKind
 
+// The 3D transform of every lz x ly x lx box of an array of boxes, sides 16 to
+// 64, up to BOX_F32_MAX or BOX_F64_MAX points, one workgroup per box
+// (fft_box.hip).  FP64: no weights.  0 on success, -1 for an unsupported shape
+// or grid, -2 on a launch error.  In place allowed.
+struct BoxArgs {
+  const void* in;
+  void* out;
+  unsigned long long nboxes;
+  const void* tw_z;              // Stockham twiddles of each axis
+  const void* tw_y;
+  const void* tw_x;
+  const float* w_load;           // optional real weights (see PassArgs)
+  const float* w_store;
+  unsigned long long w_mask;
+  int inverse;
+};
+constexpr long long BOX_F32_MAX = 16384, BOX_F64_MAX = 8192;
+constexpr unsigned long long BOX_MAX_COUNT = 0xFFFFFFFFull / 1024;  // grid size in work-items is 32-bit
+int launch_fft_box(int lz, int ly, int lx, const BoxArgs& a, void* stream, int prec);
+bool box_supported(long long lz, long long ly, long long lx, int prec);
+
 // The l-point transform (l = 4096 or 2048) along the second-fastest axis of
 // blocks of l rows of lx elements (fft_col.hip): element (o, row, x) at o * in_o
 // + row * lx + x.  l / 2048 workgroups per group of 16 adjacent columns.

@@ -14,9 +14,10 @@ namespace fftamd {
 // MODE_PLANE: fused x+y pass over whole planes (fft_xy.hip for 256 x 256,
 // fft_plane.hip for smaller ones); MODE_COL: a 4096- or 2048-point second-fastest
 // axis in one pass (fft_col.hip); MODE_CUBE_A / MODE_CUBE_B: the two passes of
-// 256 x 256 x 256 blocks with the y axis split 64 x 4 (fft_cube.hip)
+// 256 x 256 x 256 blocks with the y axis split 64 x 4 (fft_cube.hip); MODE_BOX:
+// all three axes of small boxes in one pass (fft_box.hip)
 enum PassMode { MODE_CONTIG = 0, MODE_STRIDED = 1, MODE_PLANE = 2, MODE_COL = 3, MODE_CUBE_A = 4,
-                MODE_CUBE_B = 5 };
+                MODE_CUBE_B = 5, MODE_BOX = 6 };
 // EPI_TWIDDLE multiplies point k of column c by W_M^{(c >> cshift) * k}
 // (four-step split of a long axis); EPI_BITREV stores point k at bitrev(k).
 // EPI_TWIDDLE_T is EPI_TWIDDLE of a strided pass whose output lines are

@@ -26,6 +26,7 @@ void preload_plane();
 void preload_multi();
 void preload_flow();
 void preload_wgrad();
+void preload_box();
 inline void preload_kernel(const void* f) {
   hipFuncAttributes fa;
   (void)hipFuncGetAttributes(&fa, f);

@@ -209,7 +209,8 @@ int fftamd_profile_end(char *json_out, int cap);
  * column count, middle extent, middle bit-reversal bits, outer extent,
  * four-step modulus, column shift, source and destination buffer, columns
  * per workgroup, threads per workgroup) followed by one final-copy flag.
- * Modes: 0 contiguous lines, 1 strided lines, 2 plane pass (the 2D transform
+ * Modes: 0 contiguous lines, 1 strided lines, 6 box pass (the 3D transform of every
+ * box of column-count planes of middle-extent rows x 2^log2-length columns), 2 plane pass (the 2D transform
  * of every plane of middle-extent rows x 2^log2-length columns; outer extent
  * = planes, outer stride = plane size).
  * prec: 0 FP32, 1 FP64.  With out == NULL returns the pass count; otherwise
