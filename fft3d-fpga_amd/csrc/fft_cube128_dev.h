@@ -73,21 +73,30 @@ __device__ __forceinline__ void cube128_a_tile(const CubeArgs& a, unsigned long 
   const int c = tid >> 3, tau = tid & 7;
   cpx<R> v[16];
   {
-    constexpr int RAD = sched_radix(C1_L, 0), NB = 16 / RAD;
-    const long long row = (long long)(res + 4 * c) * C1_L;
+    using D = RowDeal<C1_L, 32>;
+    constexpr int RAD = D::RAD, NB = 16 / RAD;
 #pragma unroll
     for (int bb = 0; bb < NB; ++bb)
 #pragma unroll
       for (int r = 0; r < RAD; ++r) {
-        const long long e = row + tau + C1Row::TPL * bb + r * (C1_L / RAD);
+        const long long e = (long long)(res + 4 * D::row(tid, bb)) * C1_L + D::j(tid, bb) + r * D::J;
         cpx<R> s = in[e];
         if (WL) s = cscale(s, (R)a.w_load[(unsigned long long)(base + e) & a.w_mask]);
         v[bb * RAD + r] = INV ? cswap(s) : s;
       }
   }
   static_assert(sched_np(C1_L) == 2 && sched_ns(C1_L, 1) == C1Row::TPL, "radix 8, then radix 16 ending with point tau + 8 r");
-  stage_compute<R, C1_L, MODE_CONTIG, 0, false, 32>(v, tau, nullptr);  // radix 8, no twiddles
-  stage_store_lds<R, C1_L, MODE_CONTIG, 0, 32>(v, buf, c, tau);
+  {
+    using D = RowDeal<C1_L, 32>;  // radix 8, no twiddles
+    static_assert(D::on, "two butterflies per thread, dealt out over the rows");
+#pragma unroll
+    for (int bb = 0; bb < 16 / D::RAD; ++bb) {
+      dft<R, D::RAD>(v + bb * D::RAD);
+#pragma unroll
+      for (int r = 0; r < D::RAD; ++r)
+        buf[C1Row::idx(D::row(tid, bb), D::j(tid, bb) * D::RAD + r)] = v[bb * D::RAD + r];
+    }
+  }
   __syncthreads();
   stage_load_lds<R, C1_L, MODE_CONTIG, 1, 32>(v, buf, c, tau);
   // radix-16 stage over sub-transforms of span 8: twiddles W128^{tau r} from

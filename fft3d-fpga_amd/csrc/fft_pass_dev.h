@@ -106,6 +106,31 @@ __device__ __forceinline__ void stage_store_lds(const cpx<R>* v, cpx<R>* lds, in
   }
 }
 
+// First stage of contiguous rows read from HBM.  With fewer than 16 threads per
+// row (32, 64 and 128 points) its butterflies are dealt out over the tile so
+// that 16 adjacent threads take the 16 adjacent butterflies of one row: every
+// load covers whole 128-byte segments instead of 16 to 64 bytes of each row, and
+// the outputs go to LDS whichever thread held them (256 x 32^3 55.3 -> 48.9 us,
+// 400000 x 64 points bit-reversed 101.2 -> 91.4, 60000 x 128 30.3 -> 28.0).  WANT:
+// false keeps each row on its own threads.  Butterfly b of thread tid:
+template <int L, int CC, bool WANT = true>
+struct RowDeal {
+  using G = Geom<L, MODE_CONTIG, CC>;
+  static constexpr int RAD = sched_radix(L, 0), J = L / RAD;
+  static constexpr bool on = WANT && G::NP > 1 && G::TPL < 16;
+  static __device__ __forceinline__ int row(int tid, int b) {
+    return on ? (tid + b * G::NT) / J : tid / G::TPL;
+  }
+  static __device__ __forceinline__ int j(int tid, int b) {
+    return on ? tid % J : tid % G::TPL + b * G::TPL;
+  }
+  static_assert(!on || G::NT % J == 0, "a thread keeps its butterfly index in every row");
+};
+
+// the dealt-out first stage's arithmetic and LDS stores, then the other stages
+template <typename R, int L, bool SPLIT, int CC, bool AHEAD = !SPLIT, typename D = RowDeal<L, CC>>
+__device__ __forceinline__ void run_rows(cpx<R>* v, cpx<R>* lds, int tid, const cpx<R>* __restrict__ tw);
+
 // read stage-S butterfly inputs from LDS
 template <typename R, int L, int MODE, int S, int CC = geom_cols(L, MODE)>
 __device__ __forceinline__ void stage_load_lds(cpx<R>* v, const cpx<R>* lds, int c, int tau) {
@@ -155,6 +180,25 @@ __device__ __forceinline__ void run_stages(cpx<R>* v, cpx<R>* lds, int c, int ta
   }
 }
 
+template <typename R, int L, bool SPLIT, int CC, bool AHEAD, typename D>
+__device__ __forceinline__ void run_rows(cpx<R>* v, cpx<R>* lds, int tid, const cpx<R>* __restrict__ tw) {
+  using G = typename D::G;
+  const int c = tid / G::TPL, tau = tid % G::TPL;
+  if constexpr (D::on) {
+    cpx<R> pre[TW_PER_K];
+    if constexpr (AHEAD) stage_twiddles<R, L, 1>(pre, tau, tw);
+#pragma unroll
+    for (int b = 0; b < 16 / D::RAD; ++b) {
+      dft<R, D::RAD>(v + b * D::RAD);
+#pragma unroll
+      for (int r = 0; r < D::RAD; ++r) lds[G::idx(D::row(tid, b), D::j(tid, b) * D::RAD + r)] = v[b * D::RAD + r];
+    }
+    run_stages<R, L, MODE_CONTIG, 1, SPLIT, CC, AHEAD>(v, lds, c, tau, tw, pre);
+  } else {
+    run_stages<R, L, MODE_CONTIG, 0, SPLIT, CC, AHEAD>(v, lds, c, tau, tw);
+  }
+}
+
 // Where this thread's line of tile g sits (tile = column block, middle and
 // outer line index decoded from g).
 struct TileLoc {
@@ -201,6 +245,22 @@ __device__ __forceinline__ void tile_load(const PassArgs& a, const TileLoc& t, c
   constexpr int RAD = sched_radix(L, 0);
   constexpr int NB = G::PPT / RAD;
   const cpx<R>* __restrict__ in = reinterpret_cast<const cpx<R>*>(a.in) + t.in_off;
+  if constexpr (MODE == MODE_CONTIG && RowDeal<L, CC>::on) {
+    using D = RowDeal<L, CC>;
+    const int tid = t.c * G::TPL + t.tau;
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      const int d = D::row(tid, b) - t.c;  // lines from this thread's own
+      const bool active = t.col + (unsigned)d < a.ncol;
+#pragma unroll
+      for (int r = 0; r < RAD; ++r) {
+        cpx<R> x = {R(0), R(0)};
+        if (active) x = in[(long long)d * a.in_c + (D::j(tid, b) + r * D::J) * a.in_p];
+        v[b * RAD + r] = x;
+      }
+    }
+    return;
+  }
 #pragma unroll
   for (int b = 0; b < NB; ++b) {
     const int j = t.tau + b * G::TPL;
@@ -233,22 +293,27 @@ __device__ __forceinline__ void tile_finish(const PassArgs& a, const TileLoc& t,
   {
     constexpr int RAD = sched_radix(L, 0);
     constexpr int NB = PPT / RAD;
+    using D = RowDeal<L, CC>;
+    constexpr bool deal = MODE == MODE_CONTIG && D::on;
+    const int tid = c * TPL + tau;
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
-      const int j = tau + b * TPL;
+      const int j = deal ? D::j(tid, b) : tau + b * TPL;
+      const int d = deal ? D::row(tid, b) - c : 0;
 #pragma unroll
       for (int r = 0; r < RAD; ++r) {
         cpx<R> x = v[b * RAD + r];
-        if (a.w_load && active) {
+        if (a.w_load && (deal ? col + (unsigned)d < a.ncol : active)) {
           const long long p = j + r * (L / RAD);
-          x = cscale(x, (R)a.w_load[(unsigned long long)(in_off + p * a.in_p) & a.w_mask]);
+          x = cscale(x, (R)a.w_load[(unsigned long long)(in_off + d * a.in_c + p * a.in_p) & a.w_mask]);
         }
         v[b * RAD + r] = inv ? cswap(x) : x;
       }
     }
   }
 
-  run_stages<R, L, MODE, 0, SPLIT, CC>(v, lds, c, tau, tw);
+  if constexpr (MODE == MODE_CONTIG) run_rows<R, L, SPLIT, CC>(v, lds, c * TPL + tau, tw);
+  else run_stages<R, L, MODE, 0, SPLIT, CC>(v, lds, c, tau, tw);
 
   // ---- last stage: point k = j + r*NS of the line is in v[b*RAD + r]
   constexpr int RL = sched_radix(L, NP - 1);

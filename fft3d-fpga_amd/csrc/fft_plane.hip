@@ -84,22 +84,21 @@ __global__ void __launch_bounds__(LY * LX / 32, 4) k_fft_plane_halves(const Plan
   const int rc = tid / GX::TPL, rtau = tid % GX::TPL;
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
-    constexpr int RAD = sched_radix(LX, 0), NB = 16 / RAD;
+    using D = RowDeal<LX, HY>;
+    constexpr int RAD = D::RAD, NB = 16 / RAD;
     cpx<float>* v = rr[h];
-    const int row = rc + HY * h;
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
-      const int j = rtau + b * GX::TPL;
 #pragma unroll
       for (int r = 0; r < RAD; ++r) {
-        const int e = row * LX + j + r * (LX / RAD);
+        const int e = (D::row(tid, b) + HY * h) * LX + D::j(tid, b) + r * D::J;
         cpx<float> x = in[e];
         if (WL) x = cscale(x, a.w_load[(unsigned long long)(base + e) & a.w_mask]);
         v[b * RAD + r] = INV ? cswap(x) : x;
       }
     }
     if (h) __syncthreads();  // the first half's last stage has read the buffer
-    run_stages<float, LX, MODE_CONTIG, 0, false, HY, false>(v, lds, rc, rtau, reinterpret_cast<const cpx<float>*>(a.tw_x));
+    run_rows<float, LX, false, HY, false>(v, lds, tid, reinterpret_cast<const cpx<float>*>(a.tw_x));
   }
 
   // ---- columns, in two halves: thread (column c, tau), adjacent threads on adjacent columns

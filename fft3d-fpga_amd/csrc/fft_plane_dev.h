@@ -42,20 +42,21 @@ __device__ __forceinline__ void plane_tile(const PlaneArgs& a, unsigned long lon
 
   // ---- rows: thread (row c, tau); stage 0 reads its butterfly inputs from HBM
   {
-    constexpr int RAD = sched_radix(LX, 0), NB = 16 / RAD;
+    // FP32 rows of 64 points keep their threads: 160 x 64^3 244.5 us, dealt out 248.5
+    using D = RowDeal<LX, LY, LX != 64 || sizeof(R) == 8 || SPLIT>;
+    constexpr int RAD = D::RAD, NB = 16 / RAD;
     const int c = tid / GX::TPL, tau = tid % GX::TPL;
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
-      const int j = tau + b * GX::TPL;
 #pragma unroll
       for (int r = 0; r < RAD; ++r) {
-        const int e = c * LX + j + r * (LX / RAD);
+        const int e = D::row(tid, b) * LX + D::j(tid, b) + r * D::J;
         cpx<R> x = in[e];
         if (a.w_load) x = cscale(x, (R)a.w_load[(unsigned long long)(base + e) & a.w_mask]);
         v[b * RAD + r] = INV ? cswap(x) : x;
       }
     }
-    run_stages<R, LX, MODE_CONTIG, 0, SPLIT, LY>(v, lds, c, tau, reinterpret_cast<const cpx<R>*>(a.tw_x));
+    run_rows<R, LX, SPLIT, LY, !SPLIT, D>(v, lds, tid, reinterpret_cast<const cpx<R>*>(a.tw_x));
     // last stage: point k = j + r*NS of row c -> column layout
     constexpr int NPX = GX::NP;
     constexpr int RL = sched_radix(LX, NPX - 1), NSL = sched_ns(LX, NPX - 1), NBL = 16 / RL;
