@@ -833,6 +833,21 @@ static int get_plan(int rank, const size_t* dims, size_t batch, unsigned flags, 
   return 0;
 }
 
+// Blocks of one launch of the y-split pair.  From 12 FP32 128^3 blocks up the
+// array is larger than the 256 MiB Infinity Cache holds with the input's share,
+// and chunks of at most 8 blocks (128 MiB), first pass and second pass of a chunk
+// in turn, let the second pass find the first's output there: 16 blocks 201.9 ->
+// 187.9 us, 32 395 -> 356; 12 143.6 -> 140.8, but 9 in two chunks 104.9 -> 112.7;
+// chunks of 4 lose what they gain.  Not with split precision (16 blocks 220 and
+// 220 us) or FP64 (16 blocks 394 and 393, 6 149 and 153), whose passes take longer
+// than the memory, nor for 256^3 (128 MiB each: 4 blocks 436 and 429, 8 852 and 853).
+static unsigned long long cube_chunk(int n, int kind, unsigned long long blocks) {
+  constexpr unsigned long long MOST = 8, FROM = 12;
+  if (n != 128 || kind != KIND_F32 || blocks < FROM) return blocks;
+  const unsigned long long launches = (blocks + MOST - 1) / MOST;
+  return (blocks + launches - 1) / launches;
+}
+
 static int run_plan(Plan& plan, const void* din, void* dout, bool inverse, hipStream_t stream,
                     const float* w_load, const float* w_store) {
   const bool resolve = resolve_only_flag();
@@ -911,42 +926,51 @@ static int run_plan(Plan& plan, const void* din, void* dout, bool inverse, hipSt
       cur = p.dst;
       continue;
     }
-    if (p.mode == MODE_CUBE_A || p.mode == MODE_CUBE_B) {
-      const bool A = p.mode == MODE_CUBE_A;
+    if (p.mode == MODE_CUBE_A) {  // always a plan's first pass, MODE_CUBE_B its next
+      const PassDesc& pb = plan.passes[pi + 1];
+      const int n = 1 << p.lg;
+      const size_t block = (size_t)n * n * n * esz;
+      const unsigned long long blocks = p.nouter / (unsigned)n;
+      const unsigned long long chunk = cube_chunk(n, pass_kind(plan.split, plan.prec), blocks);
       CubeArgs ca{};
-      ca.in = ptr(p.src);
-      ca.out = ptr(p.dst);
-      ca.n = 1 << p.lg;
-      ca.nplanes = A ? p.nouter : p.nouter * (unsigned long long)ca.n;
-      // 512: pass A's columns are 64-point lines, pass B's z lines 4 x 128
-      if (tab_stockham(plan, ca.n == 512 ? (A ? 64 : 128) : ca.n, &ca.tw)) return -1;
+      ca.n = n;
       if (tab_direct(plan, 256, &ca.w256)) return -1;
-      if (ca.n == 512 && tab_direct(plan, 512, &ca.w512)) return -1;
-      // pass A is always the first pass of its plan; pass B takes the store
-      // weights when it is the last
-      ca.w_load = A && pi == 0 ? w_load : nullptr;
-      ca.w_store = !A && pi + 1 == plan.passes.size() ? w_store : nullptr;
+      if (n == 512 && tab_direct(plan, 512, &ca.w512)) return -1;
       ca.w_mask = (unsigned long long)plan.per - 1ULL;
       ca.inverse = inverse ? 1 : 0;
       ca.split = plan.split ? 1 : 0;
       ca.f64 = plan.prec == PREC_F64 ? 1 : 0;
       Prof& pf = P();
-      const bool prof = pf.on && !resolve && pf.used + 2 <= pf.pool.size();
-      if (prof) HIP_TRY(hipEventRecord(pf.pool[pf.used], stream));
-      const int rc = A ? launch_fft_cube_a(ca, stream) : launch_fft_cube_b(ca, stream);
-      if (prof) {
-        HIP_TRY(hipEventRecord(pf.pool[pf.used + 1], stream));
-        char lab[64];
-        snprintf(lab, sizeof(lab), "fft_cube_%s_%s%s_%d", A ? "a" : "b", ca.f64 ? "f64" : "f32",
-                 plan.split ? "_split" : "", ca.n);
-        pf.recs.push_back({lab, pf.pool[pf.used], pf.pool[pf.used + 1]});
-        pf.used += 2;
+      for (unsigned long long b0 = 0; b0 < blocks; b0 += chunk) {
+        for (int half = 0; half < 2; ++half) {
+          const bool A = half == 0;
+          const PassDesc& d = A ? p : pb;
+          ca.in = static_cast<const char*>(ptr(d.src)) + b0 * block;
+          ca.out = static_cast<char*>(ptr(d.dst)) + b0 * block;
+          ca.nplanes = std::min(chunk, blocks - b0) * (unsigned)n;
+          // 512: pass A's columns are 64-point lines, pass B's z lines 4 x 128
+          if (tab_stockham(plan, n == 512 ? (A ? 64 : 128) : n, &ca.tw)) return -1;
+          ca.w_load = A ? w_load : nullptr;
+          ca.w_store = !A && pi + 2 == plan.passes.size() ? w_store : nullptr;
+          const bool prof = pf.on && !resolve && pf.used + 2 <= pf.pool.size();
+          if (prof) HIP_TRY(hipEventRecord(pf.pool[pf.used], stream));
+          const int rc = A ? launch_fft_cube_a(ca, stream) : launch_fft_cube_b(ca, stream);
+          if (prof) {
+            HIP_TRY(hipEventRecord(pf.pool[pf.used + 1], stream));
+            char lab[64];
+            snprintf(lab, sizeof(lab), "fft_cube_%s_%s%s_%d", A ? "a" : "b", ca.f64 ? "f64" : "f32",
+                     plan.split ? "_split" : "", n);
+            pf.recs.push_back({lab, pf.pool[pf.used], pf.pool[pf.used + 1]});
+            pf.used += 2;
+          }
+          if (rc) {
+            set_error("y-split pass launch failed (n=%d, rc=%d): %s", n, rc, hipGetErrorString(hipGetLastError()));
+            return -1;
+          }
+        }
       }
-      if (rc) {
-        set_error("y-split pass launch failed (n=%d, rc=%d): %s", ca.n, rc, hipGetErrorString(hipGetLastError()));
-        return -1;
-      }
-      cur = p.dst;
+      cur = pb.dst;
+      ++pi;
       continue;
     }
     if (p.mode == MODE_COL) {
@@ -1103,12 +1127,6 @@ struct MultiPlan {
   bool inverse = false;
   std::string sig;
   size_t points = 0;
-  // mode 2 with several shape groups: one stream per group (default
-  // priority) forked from and joined back to the caller's stream, so the
-  // groups' launch chains overlap (also as parallel branches of a HIP graph)
-  std::vector<hipStream_t> aux;
-  std::vector<hipEvent_t> aux_done;
-  hipEvent_t fork_ev = nullptr;
   // mode 3 (one dataflow launch, fft_flow.hip): every transform n^3 with
   // n = 32, 64 or 128 (128^3 out of place), FP32
   bool flow_ok = false;
@@ -1120,9 +1138,6 @@ struct MultiPlan {
   unsigned* d_done = nullptr;      // finished first-pass tiles per transform
   unsigned ndone = 0;
   ~MultiPlan() {
-    for (hipStream_t s : aux) (void)hipStreamDestroy(s);
-    for (hipEvent_t e : aux_done) (void)hipEventDestroy(e);
-    if (fork_ev) (void)hipEventDestroy(fork_ev);
     if (d_passes) (void)hipFree(d_passes);
     if (d_items) (void)hipFree(d_items);
     if (d_phase) (void)hipFree(d_phase);
@@ -1486,22 +1501,6 @@ static int multi_prepare_tables(const MultiPlan* mp) {
   return 0;
 }
 
-// the streams and events of the mode-2 fork and its tables (created outside any capture)
-static int multi_prepare_fork(MultiPlan* mp) {
-  if (multi_prepare_tables(mp)) return -1;
-  if (mp->groups.size() < 2 || !mp->aux.empty()) return 0;
-  HIP_TRY(hipEventCreateWithFlags(&mp->fork_ev, hipEventDisableTiming));
-  for (size_t i = 0; i < mp->groups.size(); ++i) {
-    hipStream_t s = nullptr;
-    hipEvent_t e = nullptr;
-    HIP_TRY(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
-    mp->aux.push_back(s);
-    HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-    mp->aux_done.push_back(e);
-  }
-  return 0;
-}
-
 // The y-split pair's arguments for a 128^3 group: pass A out of place from
 // the inputs, pass B in place on the outputs (transform tables).
 static int group_cube_args(const MultiPlan* mp, const PlaneGroup& g, CubeArgs* ca, CubeArgs* cb) {
@@ -1559,13 +1558,19 @@ static int multi_group_exec(MultiPlan* mp, const PlaneGroup& g, hipStream_t stre
   if (g.cube) {
     CubeArgs ca{}, cb{};
     if (group_cube_args(mp, g, &ca, &cb)) return -1;
-    if (launch_fft_cube_a(ca, stream)) {
-      set_error("y-split pass A launch failed: %s", hipGetErrorString(hipGetLastError()));
-      return -1;
-    }
-    if (launch_fft_cube_b(cb, stream)) {
-      set_error("y-split pass B launch failed: %s", hipGetErrorString(hipGetLastError()));
-      return -1;
+    const unsigned long long chunk = cube_chunk(128, pass_kind(mp->split, PREC_F32), g.count);
+    for (unsigned long long t = 0; t < g.count; t += chunk) {
+      ca.nplanes = cb.nplanes = std::min(chunk, g.count - t) * 128;
+      if (launch_fft_cube_a(ca, stream)) {
+        set_error("y-split pass A launch failed: %s", hipGetErrorString(hipGetLastError()));
+        return -1;
+      }
+      if (launch_fft_cube_b(cb, stream)) {
+        set_error("y-split pass B launch failed: %s", hipGetErrorString(hipGetLastError()));
+        return -1;
+      }
+      ca.tab += 2 * chunk;
+      cb.tab += 2 * chunk;
     }
     return 0;
   }
@@ -1614,20 +1619,12 @@ int multi_exec(void* handle, void* stream) {
       set_error("multi-transform reset failed: %s", hipGetErrorString(hipGetLastError()));
       return -1;
     }
-    if (mp->groups.size() < 2) {
-      for (const PlaneGroup& g : mp->groups)
-        if (multi_group_exec(mp, g, hs)) return -1;
-      return 0;
-    }
-    // the groups touch disjoint transforms: each chain on its own stream
-    if (multi_prepare_fork(mp)) return -1;
-    HIP_TRY(hipEventRecord(mp->fork_ev, hs));
-    for (size_t i = 0; i < mp->groups.size(); ++i) {
-      HIP_TRY(hipStreamWaitEvent(mp->aux[i], mp->fork_ev, 0));
-      if (multi_group_exec(mp, mp->groups[i], mp->aux[i])) return -1;
-      HIP_TRY(hipEventRecord(mp->aux_done[i], mp->aux[i]));
-    }
-    for (size_t i = 0; i < mp->groups.size(); ++i) HIP_TRY(hipStreamWaitEvent(hs, mp->aux_done[i], 0));
+    // one group after the other on the caller's stream: side by side on forked
+    // streams they shared the caches and paid for the events (the 448-transform
+    // batch 733 against 700 us, 100 x 32^3 + 20 x 64^3 + 3 x 128^3 128 against 106,
+    // one transform of each 75 against 40)
+    for (const PlaneGroup& g : mp->groups)
+      if (multi_group_exec(mp, g, hs)) return -1;
     return 0;
   }
   if (mp->mode == 3) {
@@ -1832,7 +1829,7 @@ int graph_capture_multi(void** out, void** handles, int n, void* stream) {
       return -1;
     }
     if (!multi_current(static_cast<MultiPlan*>(handles[i]))) return -1;
-    if (multi_prepare_fork(static_cast<MultiPlan*>(handles[i]))) return -1;  // no creation under capture
+    if (multi_prepare_tables(static_cast<MultiPlan*>(handles[i]))) return -1;  // no creation under capture
   }
   gr->gen = st.gen;
   HIP_TRY(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
