@@ -948,8 +948,7 @@ static int run_plan(Plan& plan, const void* din, void* dout, bool inverse, hipSt
           ca.in = static_cast<const char*>(ptr(d.src)) + b0 * block;
           ca.out = static_cast<char*>(ptr(d.dst)) + b0 * block;
           ca.nplanes = std::min(chunk, blocks - b0) * (unsigned)n;
-          // 512: pass A's columns are 64-point lines, pass B's z lines 4 x 128
-          if (tab_stockham(plan, n == 512 ? (A ? 64 : 128) : n, &ca.tw)) return -1;
+          if (n != 512 && tab_stockham(plan, n, &ca.tw)) return -1;  // 512: every factor from w512
           ca.w_load = A ? w_load : nullptr;
           ca.w_store = !A && pi + 2 == plan.passes.size() ? w_store : nullptr;
           const bool prof = pf.on && !resolve && pf.used + 2 <= pf.pool.size();

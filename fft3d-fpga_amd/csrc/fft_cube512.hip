@@ -54,6 +54,33 @@ static_assert(sched_np(64) == 2 && sched_radix(64, 0) == 4, "64 = 4 x 16");
 static_assert(sched_np(128) == 2 && sched_radix(128, 0) == 8, "128 = 8 x 16");
 constexpr int C5A_LDS = C5X_LDS > C5Col::LDS_ELEMS ? C5X_LDS : C5Col::LDS_ELEMS;
 
+// v[r] *= W512^{(STEP t r) mod 512}, r = 1..15, for t uniform over the wave.  The
+// factors are read through the constant address space, by scalar loads: vector
+// loads of the second half would wait for the first half's stores (one in-order
+// counter), and the powers formed from four of them cost 11 products a thread.
+typedef const __attribute__((address_space(4))) cpx<float>* c5_const;
+template <int STEP>
+__device__ __forceinline__ void c5_twiddle(cpx<float>* v, const void* w512, int t) {
+  const c5_const w = reinterpret_cast<c5_const>(reinterpret_cast<unsigned long long>(w512));
+#pragma unroll
+  for (int r = 1; r < 16; ++r) {
+    const auto* e = &w[(STEP * t * r) & (C5_L - 1)];
+    v[r] = cmul(v[r], cpx<float>{e->x, e->y});
+  }
+}
+
+// Wave w of the workgroup starts 256 w cycles late (at most 1.6 us of the 33 us a
+// tile takes), so that a wave's loads, whole rows in pass A and whole 128-byte
+// halves of eight rows in pass B, reach the memory together instead of
+// interleaved with those of the other fifteen.  With the scalar twiddles: split
+// 1086 -> 1068 us, FP32 1003 -> 988 (twiddles alone 1084 and 1001); 64 cycles a
+// wave 1078, 512 1077, 768 1085.  The 256^3 and 128^3 pairs, two and four
+// workgroups per CU, lose by it (16 x 128^3 378 -> 385 us).
+__device__ __forceinline__ void c5_stagger() {
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  for (int i = 0; i < w; ++i) __builtin_amdgcn_s_sleep(4);
+}
+
 // One workgroup per CU: 1024 threads (128 VGPRs each), <= 148 KiB of LDS.
 template <bool INV, bool WL, bool SPLIT>
 __global__ void __launch_bounds__(C5_NT, 1) k_fft_c512_a(const CubeArgs a) {
@@ -63,11 +90,11 @@ __global__ void __launch_bounds__(C5_NT, 1) k_fft_c512_a(const CubeArgs a) {
   const unsigned long long plane = blockIdx.x >> 3;
   const int res = blockIdx.x & 7;  // residue class a of the input rows
   if (plane >= a.nplanes) return;  // uniform over the workgroup
+  c5_stagger();
   const long long base = (long long)plane * C5_PLANE;
   const cpx<float>* in = reinterpret_cast<const cpx<float>*>(a.in) + base;
   cpx<float>* out = reinterpret_cast<cpx<float>*>(a.out) + base;
   const cpx<float>* __restrict__ wdir = reinterpret_cast<const cpx<float>*>(a.w512);
-  const cpx<float>* __restrict__ tw64 = reinterpret_cast<const cpx<float>*>(a.tw);
   const int tid = threadIdx.x;
   if (tid < C5_L) w512[tid] = wdir[tid];  // read after the first barrier
   if constexpr (SPLIT) split_atab_fill(atab);
@@ -127,7 +154,8 @@ __global__ void __launch_bounds__(C5_NT, 1) k_fft_c512_a(const CubeArgs a) {
     stage_store_lds<float, 64, MODE_STRIDED, 0, 256>(u, buf, cc, tq);
     __syncthreads();
     stage_load_lds<float, 64, MODE_STRIDED, 1, 256>(u, buf, cc, tq);
-    stage_compute<float, 64, MODE_STRIDED, 1, SPLIT, 256, SPLIT>(u, tq, tw64, buf, atab);  // radix 16, W64 twiddles
+    c5_twiddle<8>(u, a.w512, tq);  // W64^{tq r}
+    wg_dft16<SPLIT, true>(u, atab);
     // column DFT point k = tq + 4 r to row 64 res + k (pass B applies W512^{res k})
     const int kx = 16 * R + (cc & 15) + 32 * (cc >> 4);
 #pragma unroll
@@ -154,11 +182,11 @@ __global__ void __launch_bounds__(C5_NT, 1) k_fft_c512_b(const CubeArgs a) {
   const int xg = 2 * (int)(((P >> 4) & 7u) | (((P >> 9) & 3u) << 3)) + (int)((b >> 3) & 1);  // 8 columns
   const unsigned long long blk = P >> 11;
   if (blk >= a.nplanes / C5_L) return;  // uniform over the workgroup
+  c5_stagger();
   const long long base = (long long)blk * C5_BLOCK + (long long)k * C5_L + 8 * xg;
   const cpx<float>* in = reinterpret_cast<const cpx<float>*>(a.in) + base;
   cpx<float>* out = reinterpret_cast<cpx<float>*>(a.out) + base;
   const cpx<float>* __restrict__ wdir = reinterpret_cast<const cpx<float>*>(a.w512);
-  const cpx<float>* __restrict__ tw128 = reinterpret_cast<const cpx<float>*>(a.tw);
   const int tid = threadIdx.x;
   if (tid < C5_L) w512[tid] = wdir[tid];  // read after the first barrier
   if constexpr (SPLIT) split_atab_fill(atab);
@@ -219,7 +247,8 @@ __global__ void __launch_bounds__(C5_NT, 1) k_fft_c512_b(const CubeArgs a) {
     stage_store_lds<float, 128, MODE_STRIDED, 0, 128>(v, buf, cz, tz);
     __syncthreads();
     stage_load_lds<float, 128, MODE_STRIDED, 1, 128>(v, buf, cz, tz);
-    stage_compute<float, 128, MODE_STRIDED, 1, SPLIT, 128, SPLIT>(v, tz, tw128, buf, atab);  // radix 16, W128 twiddles
+    c5_twiddle<4>(v, a.w512, tz);  // W128^{tz r}
+    wg_dft16<SPLIT, true>(v, atab);
     const int xx = cz & 7, kq = (cz >> 3) & 3, dd = cz >> 5;
     const long long ob = (long long)(64 * (4 * hh + dd)) * C5_L + xx;  // row k + 64 d
 #pragma unroll
@@ -251,7 +280,7 @@ void preload_c512() { preload_kernel(reinterpret_cast<const void*>(&k_fft_c512_a
 
 int launch_fft_c512_a(const CubeArgs& a, void* stream) {
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  if (a.n != C5_L || a.nplanes == 0 || a.w_store || a.tab || !a.w512 || !a.tw || (a.split && a.w_load)) return -1;
+  if (a.n != C5_L || a.nplanes == 0 || a.w_store || a.tab || !a.w512 || (a.split && a.w_load)) return -1;
   const unsigned long long blocks = a.nplanes * 8ull;
   if (blocks > 0xFFFFFFFFull / C5_NT) return -1;  // grid size in work-items is 32-bit
   const dim3 g((unsigned)blocks), t(C5_NT);
@@ -261,7 +290,7 @@ int launch_fft_c512_a(const CubeArgs& a, void* stream) {
 
 int launch_fft_c512_b(const CubeArgs& a, void* stream) {
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  if (a.n != C5_L || a.nplanes == 0 || a.nplanes % C5_L || a.w_load || a.tab || !a.w512 || !a.tw ||
+  if (a.n != C5_L || a.nplanes == 0 || a.nplanes % C5_L || a.w_load || a.tab || !a.w512 ||
       (a.split && a.w_store))
     return -1;
   const unsigned long long blocks = (a.nplanes / C5_L) * 4096ull;  // 64 k x 64 column groups per block

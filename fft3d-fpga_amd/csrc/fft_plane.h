@@ -95,8 +95,7 @@ struct CubeArgs {
   void* out;
   int n;                         // block side: 512, 256 or 128
   unsigned long long nplanes;    // n x n planes in the array (a multiple of n for pass B)
-  const void* tw;                // Stockham twiddles of n-point lines (n = 512: of the
-                                 // 64-point lines of pass A, the 128-point lines of pass B)
+  const void* tw;                // Stockham twiddles of n-point lines (not read for n = 512)
   const void* w256;              // W256^m, m = 0..255 (in the values' precision)
   const void* w512;              // W512^m, m = 0..511 (n = 512)
   const float* w_load;
