@@ -1551,6 +1551,19 @@ static int group_plane_args(const MultiPlan* mp, const PlaneGroup& g, PlaneArgs*
   return 0;
 }
 
+// Transforms of one plane and one z launch of a shape group: all of them up to
+// the 256 MiB of the Infinity Cache, chunks of at most 160 MiB past it, whose z
+// launch then finds part of the planes there (448 uneven 659 -> 653 us, 200 x 64^3
+// 306.5 -> 297.5, 300 x 32^3 + 130 x 64^3 256 -> 249; chunks of 112 MiB 656, 300 and
+// 258.5, of 64 MiB 681, 340 and 283: every further pair of launches costs 10 us).
+// Split precision keeps one launch, its passes take longer than the memory.
+static unsigned long long plane_group_chunk(const PlaneGroup& g, bool split) {
+  const unsigned long long bytes = 8ull * g.ppt * g.ly * g.lx, most = std::max(1ull, (160ull << 20) / bytes);
+  if (split || g.count * bytes <= (256ull << 20)) return g.count;
+  const unsigned long long launches = (g.count + most - 1) / most;
+  return (g.count + launches - 1) / launches;
+}
+
 // x and y of one shape group as one plane-kernel launch, then its z axis as
 // one strided line pass over all its transforms, in place
 static int multi_group_exec(MultiPlan* mp, const PlaneGroup& g, hipStream_t stream) {
@@ -1576,16 +1589,23 @@ static int multi_group_exec(MultiPlan* mp, const PlaneGroup& g, hipStream_t stre
   PlaneArgs a{};
   PassArgs z{};
   if (group_plane_args(mp, g, &a, &z)) return -1;
-  if (launch_fft_plane(g.ly, g.lx, a, stream, mp->split)) {
-    set_error("plane kernel launch failed: %s", hipGetErrorString(hipGetLastError()));
-    return -1;
-  }
   const long long L = g.ppt;
-  // split precision applies to lines with a radix-16 stage, as in the line passes
-  if (launch_fft_pass(PREC_F32, ilog2c(L), MODE_STRIDED, EPI_NONE, z, (unsigned long long)z.ncb * g.count,
-                      stream, mp->split && L >= 16)) {
-    set_error("z pass launch failed: %s", hipGetErrorString(hipGetLastError()));
-    return -1;
+  const unsigned long long chunk = plane_group_chunk(g, mp->split);
+  for (unsigned long long t = 0; t < g.count; t += chunk) {
+    const unsigned long long n = std::min<unsigned long long>(chunk, g.count - t);
+    a.nplanes = n * g.ppt;
+    if (launch_fft_plane(g.ly, g.lx, a, stream, mp->split)) {
+      set_error("plane kernel launch failed: %s", hipGetErrorString(hipGetLastError()));
+      return -1;
+    }
+    // split precision applies to lines with a radix-16 stage, as in the line passes
+    if (launch_fft_pass(PREC_F32, ilog2c(L), MODE_STRIDED, EPI_NONE, z, (unsigned long long)z.ncb * n, stream,
+                        mp->split && L >= 16)) {
+      set_error("z pass launch failed: %s", hipGetErrorString(hipGetLastError()));
+      return -1;
+    }
+    a.tab += 2 * chunk;
+    z.tab += 2 * chunk;
   }
   return 0;
 }

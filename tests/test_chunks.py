@@ -54,3 +54,23 @@ def test_grouped_blocks_equal_single_blocks(gpu_lib, inverse):
     for s, n in zip(shapes, sizes):
         assert torch.equal(out[at:at + n].view(s), gpu_lib.c2c_dev(x[at:at + n].view(s), 3, inverse=inverse))
         at += n
+
+
+@pytest.mark.parametrize("n64", [128, 129, 161])
+def test_grouped_planes_equal_single_transforms(gpu_lib, n64):
+    """64^3 groups up to and past 256 MiB (one launch pair, then chunks), between
+    members of other shapes."""
+    import torch
+    from fftfpga_amd.multi import MultiPlan
+    shapes = [(32, 32, 32)] * 5 + [(64, 64, 64)] * (n64 - 1) + [(32, 64, 64), (64, 64, 64)]
+    sizes = [s[0] * s[1] * s[2] for s in shapes]
+    x = _input(-(-sum(sizes) // N ** 3), n64).view(-1)[:sum(sizes)].contiguous()
+    out = torch.empty_like(x)
+    plan = MultiPlan(shapes, x, out)
+    assert plan.schedule()["mode"] == 2
+    plan()
+    plan.check()
+    at = 0
+    for s, n in zip(shapes, sizes):
+        assert torch.equal(out[at:at + n].view(s), gpu_lib.c2c_dev(x[at:at + n].view(s), 3)), (at, s)
+        at += n
