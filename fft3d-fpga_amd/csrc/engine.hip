@@ -520,6 +520,41 @@ static int build_plan(int rank, const size_t* dims, size_t batch, unsigned flags
     top = -1;
   }
 
+  // planes of 65536 points and more (other than 256 x 256), out of place: two
+  // passes with the y axis split between them instead of three line passes
+  const int yr = rank == 3 && top == rank - 1 && prec == PREC_F32 && !plan.split && !aliased &&
+                         !(flags & (FLAG_NO_PLANE_FUSION | FLAG_NO_CUBE_SPLIT))
+                     ? yz_split((long long)dims[0], (long long)dims[1], (long long)dims[2])
+                     : 0;
+  if (yr && batch * dims[0] * (unsigned)yr <= PLANE_MAX_COUNT &&
+      batch * (tot / dims[0] / (unsigned)yr / 16) <= PLANE_MAX_COUNT) {
+    const long long NY = (long long)dims[1], LX = (long long)dims[2], LY = NY / yr;
+    PassDesc A;
+    A.lg = ilog2c(LX);
+    A.mode = MODE_YA;
+    A.transposing = true;  // residue a's output rows are other residues' input rows
+    A.in_p = A.out_p = 1;
+    A.in_c = A.out_c = LX;
+    A.ncol = (unsigned)LY;
+    A.K = (unsigned)LY;
+    A.nouter = batch * dims[0] * (unsigned)yr;
+    A.in_o = A.out_o = LY * LX;
+    A.M = yr;
+    ps.push_back(A);
+    PassDesc B;
+    B.lg = ilog2c((long long)dims[0]);
+    B.mode = MODE_YB;
+    B.in_p = B.out_p = NY * LX;
+    B.in_c = B.out_c = 1;
+    B.ncol = (unsigned)LX;
+    B.K = (unsigned)LY;
+    B.nouter = batch;
+    B.in_o = B.out_o = (long long)tot;
+    B.M = yr;
+    ps.push_back(B);
+    top = -1;
+  }
+
   // planes of the two fastest axes in one fused x+y pass: 256 x 256 (four
   // workgroups per plane, out of place) or up to 128 x 128 (one workgroup
   // per plane in LDS, in place allowed)
@@ -862,13 +897,14 @@ static int run_plan(Plan& plan, const void* din, void* dout, bool inverse, hipSt
   int cur = B_IN;
   for (size_t pi = 0; pi < plan.passes.size(); ++pi) {
     const PassDesc& p = plan.passes[pi];
-    if (p.mode == MODE_PLANE) {
+    if (p.mode == MODE_PLANE || p.mode == MODE_YA) {
       const int LX = 1 << p.lg, LY = (int)p.K;
       PlaneArgs xa{};
       xa.in = ptr(p.src);
       xa.out = ptr(p.dst);
       xa.nplanes = p.nouter;
       xa.plane_stride = p.in_o;
+      xa.rsplit = p.mode == MODE_YA ? (int)p.M : 0;
       if (sched_np(LX) > 1 && tab_stockham(plan, LX, &xa.tw_x)) return -1;
       if (sched_np(LY) > 1 && tab_stockham(plan, LY, &xa.tw_y)) return -1;
       xa.w_load = pi == 0 ? w_load : nullptr;
@@ -890,6 +926,42 @@ static int run_plan(Plan& plan, const void* din, void* dout, bool inverse, hipSt
       }
       if (rc) {
         set_error("plane pass launch failed (rc=%d): %s", rc, hipGetErrorString(hipGetLastError()));
+        return -1;
+      }
+      cur = p.dst;
+      continue;
+    }
+    if (p.mode == MODE_YB) {
+      YzArgs ya{};
+      ya.in = ptr(p.src);
+      ya.out = ptr(p.dst);
+      ya.nz = 1 << p.lg;
+      ya.r = (int)p.M;
+      ya.ly = p.K;
+      ya.lx = p.ncol;
+      ya.nblocks = p.nouter;
+      if (sched_np(ya.nz) > 1 && tab_stockham(plan, ya.nz, &ya.tw)) return -1;
+      if (tab_direct(plan, 512, &ya.w512)) return -1;
+      ya.wstep = 512u / (p.K * (unsigned)p.M);
+      ya.w_store = w_store;
+      ya.w_mask = (unsigned long long)plan.per - 1ULL;
+      ya.inverse = inverse ? 1 : 0;
+      // 256 MiB: 64 x 512 x 512 twice 257 -> 239 us, 128 x 512 x 256 twice 218 -> 204;
+      // one of each, 128 MiB, part of it still in the Infinity Cache: 118 -> 125, 100 -> 101
+      ya.stream = plan.total * esz > (192u << 20);
+      Prof& pf = P();
+      const bool prof = pf.on && !resolve && pf.used + 2 <= pf.pool.size();
+      if (prof) HIP_TRY(hipEventRecord(pf.pool[pf.used], stream));
+      const int rc = launch_fft_yz(ya, stream);
+      if (prof) {
+        HIP_TRY(hipEventRecord(pf.pool[pf.used + 1], stream));
+        char lab[64];
+        snprintf(lab, sizeof(lab), "fft_yz_f32_%dx%d", ya.nz, ya.r);
+        pf.recs.push_back({lab, pf.pool[pf.used], pf.pool[pf.used + 1]});
+        pf.used += 2;
+      }
+      if (rc) {
+        set_error("y-split z pass launch failed (rc=%d): %s", rc, hipGetErrorString(hipGetLastError()));
         return -1;
       }
       cur = p.dst;
@@ -1957,6 +2029,7 @@ int runtime_init(int dev, bool svm) {
   preload_flow();
   preload_wgrad();
   preload_box();
+  preload_yz();
   st.dev = dev;
   st.svm = svm;
   st.ready = true;
@@ -2079,13 +2152,16 @@ int describe_plan(int rank, const size_t* dims, size_t batch, unsigned flags, in
                        d.in_k, d.out_k, d.in_o, d.out_o, d.ncol, d.K, d.kbits,
                        (long long)d.nouter, d.M, d.cshift, d.src, d.dst,
                        d.mode == MODE_BOX ? 1
+                       : d.mode == MODE_YA ? (long long)d.K
+                       : d.mode == MODE_YB ? 16
                        : d.mode == MODE_PLANE ? (d.K == 256 && d.lg == 8 ? 64 : (long long)d.K)
                        : d.mode == MODE_COL ? 16
                        : d.mode == MODE_CUBE_A ? (d.lg == 9 ? 64 : (1LL << d.lg) / 4)   // rows per workgroup
                        : d.mode == MODE_CUBE_B ? (d.lg == 9 ? 8 : d.lg == 8 || prec == PREC_F64 ? 16 : 32)   // columns per workgroup (x 8 or 4 rows x n planes)
                        : pass_cols(d, p.split, prec),
                        d.mode == MODE_BOX ? (long long)d.ncol * (long long)(d.K << d.lg) / 16
-                       : d.mode == MODE_PLANE ? plane_threads(d)
+                       : d.mode == MODE_YB ? d.M << d.lg
+                       : d.mode == MODE_PLANE || d.mode == MODE_YA ? plane_threads(d)
                        : d.mode == MODE_COL ? 1024
                        : d.mode == MODE_CUBE_A ? (d.lg == 9 ? 1024 : d.lg == 8 ? 512 : 256)
                        : d.mode == MODE_CUBE_B ? (d.lg == 9 ? 1024 : prec == PREC_F64 ? 256 : 512)

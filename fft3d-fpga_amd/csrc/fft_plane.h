@@ -21,6 +21,11 @@ struct PlaneArgs {
   // starts at b * plane_stride in both
   const unsigned long long* tab;
   unsigned ppt;
+  // 4, 8 or 16: plane b is made of the rows a + rsplit y, a = b mod rsplit, of
+  // plane b / rsplit of the array (rsplit LY rows), read there and written as a
+  // plane of its own, rows LY a + k; out of place, LX >= 128, FP32 planes of 16384
+  // points and more.  0: plain planes
+  int rsplit;
 };
 
 // 256 x 256 planes, four workgroups per plane (fft_xy.hip).  0 on success, -1
@@ -113,6 +118,41 @@ int launch_fft_cube_a(const CubeArgs& a, void* stream);
 int launch_fft_cube_b(const CubeArgs& a, void* stream);
 int launch_fft_c512_a(const CubeArgs& a, void* stream);  // n = 512 (fft_cube512.hip)
 int launch_fft_c512_b(const CubeArgs& a, void* stream);
+
+// Boxes of nz x (ly r) x lx whose y axis is split r x ly: the second pass, after
+// a plane pass with rsplit = r (fft_yz.hip).  In place allowed.  0 on success, -1
+// for an unsupported shape or grid, -2 on a launch error.
+struct YzArgs {
+  const void* in;
+  void* out;
+  int nz, r;
+  unsigned ly, lx;
+  unsigned long long nblocks;
+  const void* tw;                // Stockham twiddles of nz-point lines
+  const void* w512;              // W512^m, m = 0..511; W_{ly r}^t = W512^{wstep t}
+  unsigned wstep;
+  const float* w_store;          // optional real weights (see PassArgs)
+  unsigned long long w_mask;
+  int inverse;
+  int stream;                    // non-temporal stores: for arrays that outgrow the caches
+};
+constexpr bool yz_tile_ok(int nz, int r) { return nz >= 16 && nz <= 256 && nz * r <= 1024; }
+// How many ways the y axis of an nz x ny x nx box is split: so that the first
+// pass has planes of 16384 points (two workgroups per CU); 0 where there is no
+// such pair.  Planes of up to 32768 points have a plane pass of their own, 256 x
+// 256 ones the four-workgroup one.  Against three line passes, at any batch (the
+// smallest, one box of 16 x 128 x 512, 23.4 -> 21.5 us): 4 x (64 x 512 x 128) 151 ->
+// 100 us, 2 x (128 x 512 x 256) 289 -> 218, 4 x (64 x 128 x 512) 141 -> 109, 64 x 512 x
+// 512 142 -> 118.  First-pass planes of 32768 points, which would take deeper
+// boxes, gained nothing: 256 x 256 x 512 278 and 284, 128 x 512 x 512 287 and 288.
+constexpr int yz_split(long long nz, long long ny, long long nx) {
+  if (nx < 128 || nx > 512 || ny < 128 || ny > 512 || (nx & (nx - 1)) || (ny & (ny - 1)) || (nz & (nz - 1)) || nz < 16 ||
+      nz > 256 || ny * nx < 65536 || (ny == 256 && nx == 256))
+    return 0;
+  const int r = (int)(ny * nx / 16384);
+  return yz_tile_ok((int)nz, r) ? r : 0;
+}
+int launch_fft_yz(const YzArgs& a, void* stream);
 
 // gw[i] = sum_b Re(conj(g[b][i]) f[b][i]) for FP32 complex g, f of batch x
 // points values (fft_wgrad.hip).  0 on success, -1 when the grid does not fit,

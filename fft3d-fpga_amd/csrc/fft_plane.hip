@@ -60,8 +60,9 @@ struct HalfGeom {
                 "points tau + TPL r: r < 8 are columns 0 .. LX/2 - 1");
 };
 
-// WL, WS: the launch carries load or store weights.
-template <int LY, int LX, bool INV, bool WL, bool WS>
+// WL, WS: the launch carries load or store weights.  RS: planes of every rsplit-th
+// row (see PlaneArgs), the first pass of a box with larger planes.
+template <int LY, int LX, bool INV, bool WL, bool WS, bool RS = false>
 __global__ void __launch_bounds__(LY * LX / 32, 4) k_fft_plane_halves(const PlaneArgs a) {
   using HG = HalfGeom<LY, LX>;
   using GX = typename HG::GX;
@@ -74,6 +75,11 @@ __global__ void __launch_bounds__(LY * LX / 32, 4) k_fft_plane_halves(const Plan
     const unsigned t = (unsigned)(plane / a.ppt), z = (unsigned)(plane % a.ppt);
     base = (long long)a.tab[2 * t] + (long long)z * (LY * LX);
     obase = (long long)a.tab[2 * t + 1] + (long long)z * (LY * LX);
+  }
+  const int rstride = RS ? a.rsplit * LX : LX;  // between the plane's rows
+  if (RS) {
+    const long long res = (long long)(plane & (unsigned)(a.rsplit - 1));
+    base = ((long long)plane - res) * (LY * LX) + res * LX;
   }
   const cpx<float>* __restrict__ in = reinterpret_cast<const cpx<float>*>(a.in) + base;
   cpx<float>* __restrict__ out = reinterpret_cast<cpx<float>*>(a.out) + obase;
@@ -91,7 +97,7 @@ __global__ void __launch_bounds__(LY * LX / 32, 4) k_fft_plane_halves(const Plan
     for (int b = 0; b < NB; ++b) {
 #pragma unroll
       for (int r = 0; r < RAD; ++r) {
-        const int e = (D::row(tid, b) + HY * h) * LX + D::j(tid, b) + r * D::J;
+        const int e = (D::row(tid, b) + HY * h) * rstride + D::j(tid, b) + r * D::J;
         cpx<float> x = in[e];
         if (WL) x = cscale(x, a.w_load[(unsigned long long)(base + e) & a.w_mask]);
         v[b * RAD + r] = INV ? cswap(x) : x;
@@ -133,9 +139,19 @@ __global__ void __launch_bounds__(LY * LX / 32, 4) k_fft_plane_halves(const Plan
   }
 }
 
+// shapes that yz_split leaves the first pass
+constexpr bool rsplit_shape(int ly, int lx) { return lx >= 128 && ly * lx == 16384; }
+
 template <int LY, int LX, bool INV>
 static void launch_halves(const PlaneArgs& a, hipStream_t s) {
   const dim3 grid((unsigned)a.nplanes), block(HalfGeom<LY, LX>::NT);
+  if constexpr (rsplit_shape(LY, LX)) {
+    if (a.rsplit) {
+      if (a.w_load) FFTAMD_LAUNCH((k_fft_plane_halves<LY, LX, INV, true, false, true>), grid, block, 0, s, a);
+      else FFTAMD_LAUNCH((k_fft_plane_halves<LY, LX, INV, false, false, true>), grid, block, 0, s, a);
+      return;
+    }
+  }
   if (a.w_load) {
     if (a.w_store) FFTAMD_LAUNCH((k_fft_plane_halves<LY, LX, INV, true, true>), grid, block, 0, s, a);
     else FFTAMD_LAUNCH((k_fft_plane_halves<LY, LX, INV, true, false>), grid, block, 0, s, a);
@@ -216,6 +232,9 @@ int launch_fft_plane(int ly, int lx, const PlaneArgs& a, void* stream, bool spli
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   if (!plane_shape_ok(ly, lx, pass_kind(split, prec)) || (prec == PREC_F64 && (split || a.w_load || a.w_store)) || a.nplanes == 0 || a.nplanes > 0xFFFFFFFFull / 1024 ||
       (a.tab && a.ppt == 0))
+    return -1;
+  if (a.rsplit && (!rsplit_shape(ly, lx) || prec != PREC_F32 || split || a.tab || a.w_store || a.plane_stride != (long long)ly * lx ||
+                   (a.rsplit != 4 && a.rsplit != 8 && a.rsplit != 16) || a.nplanes % (unsigned)a.rsplit))
     return -1;
   const bool ok = prec == PREC_F64 ? dispatch_ly<false, double>(ly, lx, a, s)
                   : split           ? dispatch_ly<true>(ly, lx, a, s)

@@ -17,7 +17,7 @@ namespace fftamd {
 // 256 x 256 x 256 blocks with the y axis split 64 x 4 (fft_cube.hip); MODE_BOX:
 // all three axes of small boxes in one pass (fft_box.hip)
 enum PassMode { MODE_CONTIG = 0, MODE_STRIDED = 1, MODE_PLANE = 2, MODE_COL = 3, MODE_CUBE_A = 4,
-                MODE_CUBE_B = 5, MODE_BOX = 6 };
+                MODE_CUBE_B = 5, MODE_BOX = 6, MODE_YA = 7, MODE_YB = 8 };
 // EPI_TWIDDLE multiplies point k of column c by W_M^{(c >> cshift) * k}
 // (four-step split of a long axis); EPI_BITREV stores point k at bitrev(k).
 // EPI_TWIDDLE_T is EPI_TWIDDLE of a strided pass whose output lines are

@@ -27,6 +27,7 @@ void preload_multi();
 void preload_flow();
 void preload_wgrad();
 void preload_box();
+void preload_yz();
 inline void preload_kernel(const void* f) {
   hipFuncAttributes fa;
   (void)hipFuncGetAttributes(&fa, f);
