@@ -25,9 +25,11 @@ constexpr int kind_of(bool split) { return pass_kind(split, sizeof(R) == 4 ? PRE
 template <typename R, int L, int MODE, int EPI, bool SPLIT, int DIR, int CC>
 __global__ void __launch_bounds__(CC * geom_tpl(L)) k_fft_pass(const PassArgs a) {
   using G = Geom<L, MODE, CC>;
-  constexpr bool NEED_LDS = G::NP > 1 || EPI == EPI_TWIDDLE_T;
+  constexpr bool ROWS16 = L == 16 && MODE == MODE_CONTIG;
+  constexpr bool NEED_LDS = G::NP > 1 || EPI == EPI_TWIDDLE_T || ROWS16;
   __shared__ cpx<R> lds[NEED_LDS ? G::LDS_ELEMS : 1];
-  pass_block<R, L, MODE, EPI, SPLIT, DIR, CC>(a, blockIdx.x, lds, (int)threadIdx.x);
+  if constexpr (ROWS16) rows16_block<R, EPI, SPLIT, DIR, CC>(a, blockIdx.x, lds, (int)threadIdx.x);
+  else pass_block<R, L, MODE, EPI, SPLIT, DIR, CC>(a, blockIdx.x, lds, (int)threadIdx.x);
 }
 
 // ---- launch table ------------------------------------------------------------
