@@ -54,9 +54,9 @@ constexpr int geom_tpl(int L) { return L / geom_ppt(L); }
 // Lines per workgroup.  Contiguous lines: 256 threads per workgroup (one line
 // per workgroup from L = 4096 up).  Strided lines: at least 16 adjacent
 // columns (128-byte row segments; narrower segments measured far slower) and
-// 256 threads up to L = 256; 32 columns (256-byte segments, 1024 threads) at
-// L = 512, where rows lie 4 KiB to 2 MiB apart (measured 7-18% faster than 16
-// on the y and z passes of a 512^3 array; slower at L = 256); 16 columns
+// 256 threads up to L = 256; at L = 512 32 columns (256-byte segments, 1024
+// threads; measured 7-18% faster than 16 on the y and z passes of a 512^3 array,
+// slower at L = 256) for large launches, see geom_cols_launch; 16 columns
 // (1024 threads) at L = 1024, the four-step passes of long 1D axes.
 constexpr int geom_cols(int L, int mode) {
   return mode == MODE_CONTIG ? (geom_tpl(L) >= 256 ? 1 : 256 / geom_tpl(L))
@@ -89,14 +89,19 @@ constexpr int geom_cols_tiny(int L, int mode, int kind) {
 // gives at most half of the 256 CUs a workgroup, then `tiny` below 64 workgroups.
 // Measured for both passes of natural-order 1D transforms: 2^18 points (16
 // workgroups of 32 columns) 20.9 us, of 8 columns 14.2; 2^21 (128 of 32 in its
-// first pass) 37.3 us, of 16 columns 35.2; 12 x 2^18 (192 of 32) 29.1 us, of 16
-// columns 30.0, of 8 36.0; 2^20 (64 of 16) 25.0 us, of 8 24.6; 3 x 2^20 (192 of
-// 16) 29.1 us, of 8 36.8.  Contiguous 1024-point lines, 100 of them (25
-// workgroups of four): 10.9 us, one per workgroup 9.8.
+// first pass) 37.3 us, of 16 columns 35.2; 12 x 2^18 of 16 columns 29.1 us, of 8
+// 36.0; 2^20 (64 of 16) 25.0 us, of 8 24.6; 3 x 2^20 (192 of 16) 29.1 us, of 8
+// 36.8.  Contiguous 1024-point lines, 100 of them (25 workgroups of four): 10.9
+// us, one per workgroup 9.8.
+// FP32 strided lines of 512 points take 16 columns, two workgroups per CU instead
+// of one of 1024 threads, up to 512 MiB: 60 x 2^18 points 120.4 -> 103.8 us, 8 x (512 x
+// 256 x 16) 99.9 -> 92.3, 8 x (512 x 4096) 102.5 -> 93.2, 256 MiB 2 x (512 x 256 x 128)
+// 248.5 -> 246.4; past the caches 1000 x (512 x 256), 1 GiB, 797 -> 831.
 constexpr int geom_cols_launch(int L, int mode, int kind, unsigned long long lines) {
   int c = geom_cols_for(L, mode, kind);
   const int mid = geom_cols_mid(L, mode, kind), tiny = geom_cols_tiny(L, mode, kind);
-  if (mid && lines <= 128ull * (unsigned)c) c = mid;
+  const bool l512 = L == 512 && mode == MODE_STRIDED && kind == KIND_F32;
+  if (mid && lines <= (l512 ? 131072ull : 128ull * (unsigned)c)) c = mid;
   if (tiny && lines < 64ull * (unsigned)c) c = tiny;
   return c;
 }
