@@ -591,7 +591,10 @@ static int build_plan(int rank, const size_t* dims, size_t batch, unsigned flags
     unsigned long long O = batch;
     for (int d = 0; d < rank - 2; ++d) O *= dims[d];
     const int LY = (int)dims[rank - 2];
-    if (col_supported(LY, LX, O) && (unsigned long long)(LX / 16) * O >= COL_MIN_GROUPS) {
+    // 2D arrays of 2048 rows in place take the temporary buffer: 2048 x 1024 (64 groups) 36.2
+    // against 33.5 us for the four-step pair, 3 x (2048 x 512) (96) 32.0 against 33.8
+    const unsigned long long least = LY == 2048 && rank == 2 && aliased ? 96 : COL_MIN_GROUPS;
+    if (col_supported(LY, LX, O) && (unsigned long long)(LX / 16) * O >= least) {
       ps.push_back(col_pass(LY, LX, O));
       col_axis = rank - 2;
     }
@@ -685,8 +688,13 @@ static int build_plan(int rank, const size_t* dims, size_t batch, unsigned flags
         p.ncol = (unsigned)O;
         ps.push_back(p);
       } else {
+        // split precision's tiles come in one size, too few workgroups for two
+        // strided passes over up to 2^20 points: it keeps the second half contiguous
+        // there, whose store scatters single points (2^15 points 13.0 against 16.3 us,
+        // 2^16 14.8 and 17.6, 2^20 33.2 and 37.9; 64 x 2^15 30.9 and 29.9)
+        const bool scatter = !bitrev && plan.split && (unsigned long long)L * O <= (1ull << 20);
         int lg1, lg2;
-        if ((bitrev ? split_contig(prec, lg, &lg1, &lg2) : split_natural(prec, lg, &lg1, &lg2))) {
+        if ((bitrev || scatter ? split_contig(prec, lg, &lg1, &lg2) : split_natural(prec, lg, &lg1, &lg2))) {
           set_error("contiguous axis of 2^%d points exceeds the supported length", lg);
           return -1;
         }
@@ -702,7 +710,7 @@ static int build_plan(int rank, const size_t* dims, size_t batch, unsigned flags
         A.in_o = A.out_o = L;
         A.M = L;
         A.cshift = 0;
-        if (!bitrev) {
+        if (!bitrev && !scatter) {
           // line n2 leaves the pass as the contiguous run Z[n2][k1]; the DFT
           // over n2 at stride L1 then ends in natural order, X[k1 + L1 k2] in
           // place, in whole 128-byte segments (a contiguous pass over n2 whose
@@ -721,16 +729,24 @@ static int build_plan(int rank, const size_t* dims, size_t batch, unsigned flags
         B.transposing = true;
         B.nouter = O;
         B.in_o = B.out_o = L;
-        // out[bitrev(k1)*L2 + bitrev(k2)] = X[k1 + L1 k2]: column bit reversal is
-        // expressed through the middle index, one column per K
-        B.epi = EPI_BITREV;
-        B.in_p = B.out_p = 1;
-        B.ncol = 1;
-        B.K = (unsigned)L1;
-        B.in_k = L2;
-        B.out_k = L2;
-        B.in_c = B.out_c = 0;
-        B.kbits = (unsigned)lg1;
+        B.in_p = 1;
+        if (bitrev) {
+          // out[bitrev(k1)*L2 + bitrev(k2)] = X[k1 + L1 k2]: column bit reversal is
+          // expressed through the middle index, one column per K
+          B.epi = EPI_BITREV;
+          B.out_p = 1;
+          B.ncol = 1;
+          B.K = (unsigned)L1;
+          B.in_k = L2;
+          B.out_k = L2;
+          B.in_c = B.out_c = 0;
+          B.kbits = (unsigned)lg1;
+        } else {  // X[k1 + L1 k2] at its natural position
+          B.out_p = L1;
+          B.in_c = L2;
+          B.out_c = 1;
+          B.ncol = (unsigned)L1;
+        }
         ps.push_back(B);
       }
     } else {
