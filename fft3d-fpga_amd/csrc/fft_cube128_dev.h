@@ -48,7 +48,7 @@ constexpr int C1A_TWS = 8 * 15;
 
 // Pass A tile `id` (plane id / 4, residue class id % 4) by threads tid < 256:
 // buf holds C1A_LDS elements, tws 120.
-template <bool INV, bool WL, bool SPLIT, typename R = float, bool PLAIN = false>
+template <bool INV, bool WL, bool SPLIT, typename R = float>
 __device__ __forceinline__ void cube128_a_tile(const CubeArgs& a, unsigned long long id, cpx<R>* buf, cpx<R>* tws,
                                                int tid) {
   // tws: row stage-1 twiddles W128^{k r} at [15 k + r - 1]
@@ -73,7 +73,7 @@ __device__ __forceinline__ void cube128_a_tile(const CubeArgs& a, unsigned long 
   const int c = tid >> 3, tau = tid & 7;
   cpx<R> v[16];
   {
-    using D = RowDeal<C1_L, 32, !PLAIN>;  // PLAIN as in pass_block
+    using D = RowDeal<C1_L, 32>;
     constexpr int RAD = D::RAD, NB = 16 / RAD;
 #pragma unroll
     for (int bb = 0; bb < NB; ++bb)
@@ -87,7 +87,8 @@ __device__ __forceinline__ void cube128_a_tile(const CubeArgs& a, unsigned long 
   }
   static_assert(sched_np(C1_L) == 2 && sched_ns(C1_L, 1) == C1Row::TPL, "radix 8, then radix 16 ending with point tau + 8 r");
   {
-    using D = RowDeal<C1_L, 32, !PLAIN>;  // radix 8, no twiddles
+    using D = RowDeal<C1_L, 32>;  // radix 8, no twiddles
+    static_assert(D::on, "two butterflies per thread, dealt out over the rows");
 #pragma unroll
     for (int bb = 0; bb < 16 / D::RAD; ++bb) {
       dft<R, D::RAD>(v + bb * D::RAD);

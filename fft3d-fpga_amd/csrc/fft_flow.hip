@@ -62,21 +62,21 @@ __device__ __forceinline__ void flow_tile(const FlowArgs& fa, const FlowItem& it
     const FlowGroup& g = fa.grp[0];
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     if (!it.pass)
-      plane_tile<32, 32, INV, false, float, true>(g.pa, tr * 32 + 8 * sub + w, lds + w * FLOW_P32, tid & 63);
+      plane_tile<32, 32, INV, false>(g.pa, tr * 32 + 8 * sub + w, lds + w * FLOW_P32, tid & 63);
     else
-      pass_block<float, 32, MODE_STRIDED, EPI_NONE, false, DIR, geom_cols(32, MODE_STRIDED), true>(g.za, tr * g.za.ncb + 2 * sub + half,
+      pass_block<float, 32, MODE_STRIDED, EPI_NONE, false, DIR>(g.za, tr * g.za.ncb + 2 * sub + half,
                                                                  lds + half * FlowZ32::LDS_ELEMS, h);
   } else if (it.group == 1) {  // 64^3
     const FlowGroup& g = fa.grp[1];
     if (!it.pass)
-      plane_tile<64, 64, INV, false, float, true>(g.pa, tr * 64 + 2 * sub + half, lds + half * FLOW_P64, h);
+      plane_tile<64, 64, INV, false>(g.pa, tr * 64 + 2 * sub + half, lds + half * FLOW_P64, h);
     else
-      pass_block<float, 64, MODE_STRIDED, EPI_NONE, false, DIR, geom_cols(64, MODE_STRIDED), true>(g.za, tr * g.za.ncb + 2 * sub + half,
+      pass_block<float, 64, MODE_STRIDED, EPI_NONE, false, DIR>(g.za, tr * g.za.ncb + 2 * sub + half,
                                                                  lds + half * FlowZ64::LDS_ELEMS, h);
   } else {  // 128^3
     const FlowGroup& g = fa.grp[2];
     if (!it.pass)
-      cube128_a_tile<INV, false, false, float, true>(g.ca, tr * 512 + 2 * sub + half, lds + half * FLOW_CA,
+      cube128_a_tile<INV, false, false>(g.ca, tr * 512 + 2 * sub + half, lds + half * FLOW_CA,
                                         lds + half * FLOW_CA + C1A_BUF, h);
     else
       cube128_b_tile<INV, false, false>(g.cb, (unsigned)(tr * 128 + sub), lds, nullptr, tid);

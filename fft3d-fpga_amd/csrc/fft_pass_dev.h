@@ -239,14 +239,14 @@ __device__ __forceinline__ TileLoc tile_locate(const PassArgs& a, unsigned long 
 
 // Raw stage-0 inputs of this thread straight from HBM (no arithmetic, so a
 // pipelined kernel can issue them one tile ahead).
-template <typename R, int L, int MODE, int CC = geom_cols(L, MODE), bool PLAIN = false>
+template <typename R, int L, int MODE, int CC = geom_cols(L, MODE)>
 __device__ __forceinline__ void tile_load(const PassArgs& a, const TileLoc& t, cpx<R>* v) {
   using G = Geom<L, MODE, CC>;
   constexpr int RAD = sched_radix(L, 0);
   constexpr int NB = G::PPT / RAD;
   const cpx<R>* __restrict__ in = reinterpret_cast<const cpx<R>*>(a.in) + t.in_off;
-  if constexpr (MODE == MODE_CONTIG && RowDeal<L, CC, !PLAIN>::on) {
-    using D = RowDeal<L, CC, !PLAIN>;
+  if constexpr (MODE == MODE_CONTIG && RowDeal<L, CC>::on) {
+    using D = RowDeal<L, CC>;
     const int tid = t.c * G::TPL + t.tau;
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
@@ -278,8 +278,7 @@ __device__ __forceinline__ void tile_load(const PassArgs& a, const TileLoc& t, c
 // whose raw inputs are in v.  DIR: 0 forward, 1 inverse (the swaps of
 // swap(DFT(swap(x))) are register renames), -1 taken from a.inverse at run
 // time (per-element selects).
-template <typename R, int L, int MODE, int EPI, bool SPLIT = false, int DIR = -1, int CC = geom_cols(L, MODE),
-          bool PLAIN = false>
+template <typename R, int L, int MODE, int EPI, bool SPLIT = false, int DIR = -1, int CC = geom_cols(L, MODE)>
 __device__ __forceinline__ void tile_finish(const PassArgs& a, const TileLoc& t, cpx<R>* v, cpx<R>* lds) {
   const bool inv = DIR < 0 ? a.inverse != 0 : DIR == 1;
   using G = Geom<L, MODE, CC>;
@@ -294,7 +293,7 @@ __device__ __forceinline__ void tile_finish(const PassArgs& a, const TileLoc& t,
   {
     constexpr int RAD = sched_radix(L, 0);
     constexpr int NB = PPT / RAD;
-    using D = RowDeal<L, CC, !PLAIN>;
+    using D = RowDeal<L, CC>;
     constexpr bool deal = MODE == MODE_CONTIG && D::on;
     const int tid = c * TPL + tau;
 #pragma unroll
@@ -313,10 +312,8 @@ __device__ __forceinline__ void tile_finish(const PassArgs& a, const TileLoc& t,
     }
   }
 
-  constexpr bool AHEAD = !SPLIT && !PLAIN;
-  if constexpr (MODE == MODE_CONTIG)
-    run_rows<R, L, SPLIT, CC, AHEAD, RowDeal<L, CC, !PLAIN>>(v, lds, c * TPL + tau, tw);
-  else run_stages<R, L, MODE, 0, SPLIT, CC, AHEAD>(v, lds, c, tau, tw);
+  if constexpr (MODE == MODE_CONTIG) run_rows<R, L, SPLIT, CC>(v, lds, c * TPL + tau, tw);
+  else run_stages<R, L, MODE, 0, SPLIT, CC>(v, lds, c, tau, tw);
 
   // ---- last stage: point k = j + r*NS of the line is in v[b*RAD + r]
   constexpr int RL = sched_radix(L, NP - 1);
@@ -431,17 +428,15 @@ __device__ __forceinline__ void tile_finish(const PassArgs& a, const TileLoc& t,
 // Geom::NT - 1.  Used by k_fft_pass (one tile per workgroup) and by the
 // persistent multi-transform kernels (which may run two tiles side by side in
 // one workgroup, each half with its own tid range and LDS, the halves made of
-// whole waves).  PLAIN: rows on their own threads and twiddles loaded where they
-// are used, for the dataflow kernel, which is at its register limit (the 448 batch
-// 878 us with the rows dealt out and the twiddles ahead, 807 without).
+// whole waves).
 template <typename R, int L, int MODE, int EPI, bool SPLIT = false, int DIR = -1,
-          int CC = geom_cols(L, MODE), bool PLAIN = false>
+          int CC = geom_cols(L, MODE)>
 __device__ __forceinline__ void pass_block(const PassArgs& a, unsigned long long g, cpx<R>* lds,
                                            int tid) {
   cpx<R> v[Geom<L, MODE, CC>::PPT];
   const TileLoc t = tile_locate<L, MODE, CC>(a, g, tid);
-  tile_load<R, L, MODE, CC, PLAIN>(a, t, v);
-  tile_finish<R, L, MODE, EPI, SPLIT, DIR, CC, PLAIN>(a, t, v, lds);
+  tile_load<R, L, MODE, CC>(a, t, v);
+  tile_finish<R, L, MODE, EPI, SPLIT, DIR, CC>(a, t, v, lds);
 }
 
 // The same for contiguous lines of 16 points, which a thread holds whole: loads

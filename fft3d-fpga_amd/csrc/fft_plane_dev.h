@@ -23,8 +23,8 @@ struct PlaneGeom {
 // One plane (index `plane` of the array, or of the transform table) by
 // threads tid = 0 .. NT - 1 with PlaneGeom::LDS elements of LDS at lds.
 // SPLIT: radix-16 stages on FP16 matrix cores with hi+lo operands
-// (fft_split.h; a tile is then made of whole waves).  PLAIN as in pass_block.
-template <int LY, int LX, bool INV, bool SPLIT, typename R = float, bool PLAIN = false>
+// (fft_split.h; a tile is then made of whole waves).
+template <int LY, int LX, bool INV, bool SPLIT, typename R = float>
 __device__ __forceinline__ void plane_tile(const PlaneArgs& a, unsigned long long plane, cpx<R>* lds,
                                            int tid) {
   using PG = PlaneGeom<LY, LX, SPLIT>;
@@ -43,7 +43,7 @@ __device__ __forceinline__ void plane_tile(const PlaneArgs& a, unsigned long lon
   // ---- rows: thread (row c, tau); stage 0 reads its butterfly inputs from HBM
   {
     // FP32 rows of 64 points keep their threads: 160 x 64^3 244.5 us, dealt out 248.5
-    using D = RowDeal<LX, LY, !PLAIN && (LX != 64 || sizeof(R) == 8 || SPLIT)>;
+    using D = RowDeal<LX, LY, LX != 64 || sizeof(R) == 8 || SPLIT>;
     constexpr int RAD = D::RAD, NB = 16 / RAD;
     const int c = tid / GX::TPL, tau = tid % GX::TPL;
     if constexpr (LX == 16) {
@@ -73,7 +73,7 @@ __device__ __forceinline__ void plane_tile(const PlaneArgs& a, unsigned long lon
         }
       }
     }
-    run_rows<R, LX, SPLIT, LY, !SPLIT && !PLAIN, D>(v, lds, tid, reinterpret_cast<const cpx<R>*>(a.tw_x));
+    run_rows<R, LX, SPLIT, LY, !SPLIT, D>(v, lds, tid, reinterpret_cast<const cpx<R>*>(a.tw_x));
     // last stage: point k = j + r*NS of row c -> column layout
     constexpr int NPX = GX::NP;
     constexpr int RL = sched_radix(LX, NPX - 1), NSL = sched_ns(LX, NPX - 1), NBL = 16 / RL;
@@ -92,7 +92,7 @@ __device__ __forceinline__ void plane_tile(const PlaneArgs& a, unsigned long lon
     const int c = tid % LX, tau = tid / LX;
     stage_load_lds<R, LY, MODE_STRIDED, 0, LX>(v, lds, c, tau);
     __syncthreads();  // every thread holds its stage-0 inputs before stage 0 stores
-    run_stages<R, LY, MODE_STRIDED, 0, SPLIT, LX, !SPLIT && !PLAIN>(v, lds, c, tau, reinterpret_cast<const cpx<R>*>(a.tw_y));
+    run_stages<R, LY, MODE_STRIDED, 0, SPLIT, LX>(v, lds, c, tau, reinterpret_cast<const cpx<R>*>(a.tw_y));
     constexpr int NPY = GY::NP;
     constexpr int RL = sched_radix(LY, NPY - 1), NSL = sched_ns(LY, NPY - 1), NBL = 16 / RL;
 #pragma unroll
