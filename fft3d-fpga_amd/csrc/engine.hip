@@ -690,8 +690,8 @@ static int build_plan(int rank, const size_t* dims, size_t batch, unsigned flags
       } else {
         // split precision's tiles come in one size, too few workgroups for two
         // strided passes over up to 2^20 points: it keeps the second half contiguous
-        // there, whose store scatters single points (2^15 points 13.0 against 16.3 us,
-        // 2^16 14.8 and 17.6, 2^20 33.2 and 37.9; 64 x 2^15 30.9 and 29.9)
+        // there, whose store scatters single points (2^15 points 11.3 against 16.3 us,
+        // 2^16 in place 14.1 and 17.6, 2^20 32.5 and 37.9; 64 x 2^15 30.9 and 29.9)
         const bool scatter = !bitrev && plan.split && (unsigned long long)L * O <= (1ull << 20);
         int lg1, lg2;
         if ((bitrev || scatter ? split_contig(prec, lg, &lg1, &lg2) : split_natural(prec, lg, &lg1, &lg2))) {

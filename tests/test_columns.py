@@ -94,7 +94,7 @@ def test_vs_oracle(gpu_lib, orc, shape, dtype, split):
         xt = base[1:].view(batch, *dims)
         y = gpu_lib.c2c_dev(xt, 2, inverse=inv, split=split)
         gpu_lib.c2c_dev(xt, 2, inverse=inv, split=split, out=xt)
-        if shape == (2048, 1024):  # in place by another route
+        if shape[-2] == 2048 and n // 2048 // 16 < 96:  # in place by another route
             assert float((xt - y).abs().pow(2).sum().sqrt() / y.abs().pow(2).sum().sqrt()) <= 2 * tol
         else:
             assert torch.equal(xt, y)
